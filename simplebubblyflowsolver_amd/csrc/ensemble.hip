@@ -81,9 +81,9 @@ struct sbfs_ensemble {
   RowArgs* rows[2] = {};     // [3 * n]
   PostArgs* post[2] = {};
   uint2* maps = nullptr;
-  unsigned nb_dt = 0, nb_march = 0, nb_row = 0, nb_mode = 0, nb_post = 0, nb_part = 0, nb_conv = 0;
-  unsigned off_march = 0, off_row = 0, off_mode = 0, off_post = 0, off_part = 0, off_conv = 0;
-  size_t lds = 0, lds_conv = 0;
+  unsigned nb_dt = 0, nb_march = 0, nb_row = 0, nb_mode = 0, nb_post = 0, nb_part = 0, nb_conv = 0, nb_col = 0;
+  unsigned off_march = 0, off_row = 0, off_mode = 0, off_post = 0, off_part = 0, off_conv = 0, off_col = 0;
+  size_t lds = 0, lds_conv = 0, lds_col = 0;
   int row_threads = 64;
   double* dts = nullptr;
   hipGraphExec_t graph[2] = {};
@@ -163,12 +163,23 @@ static int plan(sbfs_ensemble* e) {
     lds_rows = std::max(lds_rows, units * wave_lds(r.m));
   }
   e->nb_row = (unsigned)map.size() - e->off_row;
-  // tridiagonal: sequential cases by 64-mode groups; partitioned cases by
+  // tridiagonal: sequential cases by groups of whole columns in LDS, or (too
+  // long for it) by 64-mode groups; partitioned cases by
   // tiles of 64 modes x 4 chunks and by groups of the convolution's modes
   e->off_mode = (unsigned)map.size();
   for (int c = 0; c < n; c++)
-    if (steps[0][c].rows[0].L == 0) add(c, cdiv(steps[0][c].rows[0].nx, 64));
+    if (steps[0][c].rows[0].L == 0 && !tdm_columns(steps[0][c].rows[0].ny)) add(c, cdiv(steps[0][c].rows[0].nx, 64));
   e->nb_mode = (unsigned)map.size() - e->off_mode;
+  e->off_col = (unsigned)map.size();
+  e->lds_col = 0;
+  for (int c = 0; c < n; c++) {
+    const auto& r = steps[0][c].rows[0];
+    const int mw = tdm_columns(r.ny);
+    if (r.L != 0 || !mw) continue;
+    add(c, cdiv(r.nx, mw));
+    e->lds_col = std::max(e->lds_col, tdm_column_lds(r.ny, mw));
+  }
+  e->nb_col = (unsigned)map.size() - e->off_col;
   e->off_part = (unsigned)map.size();
   int pmax = 1;
   for (int c = 0; c < n; c++) {
@@ -251,6 +262,9 @@ static int launch_step(sbfs_ensemble* e, int p) {
     if (e->nb_mode)
       SBFS_TIMED("k_tdm_sequential", hipLaunchKernelGGL(k_tdm_sequential_batch, dim3(e->nb_mode), dim3(64), 0,
                                                         stream(), ro, mp + e->off_mode));
+    if (e->nb_col)
+      SBFS_TIMED("k_tdm_columns", hipLaunchKernelGGL(k_tdm_columns_batch, dim3(e->nb_col), dim3(256), e->lds_col,
+                                                     stream(), ro, mp + e->off_col));
     if (e->nb_part) {
       SBFS_TIMED("k_part_reduce", hipLaunchKernelGGL(k_part_reduce_batch, dim3(e->nb_part), dim3(64, 4), 0,
                                                      stream(), ro, mp + e->off_part));

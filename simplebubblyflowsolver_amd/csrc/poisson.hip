@@ -41,6 +41,7 @@ void poisson_destroy(PoissonPlan* p) {
   (void)hipFree(p->buf);
   (void)hipFree(p->v);
   (void)hipFree(p->q1);
+  (void)hipFree(p->cl);
   (void)hipFree(p->evals);
   (void)hipFree(p->tw);
   (void)hipFree(p->t1);
@@ -627,6 +628,207 @@ __global__ void k_tdm_sequential(double* __restrict__ q, double* __restrict__ v,
   tdm_sequential_body(q, v, q1, nx, ny, evals, l, u, pin_mode0, blockIdx.x * blockDim.x + threadIdx.x);
 }
 
+// The same solve, operation for operation, with what does not depend on the
+// data (the pivots' inverses v, the corner spike's solution q1 and the closure's
+// denominator) from tables built once per plan, and whole columns in LDS.  What
+// bounds it is the chain of ny steps per mode, three dependent FP64 operations
+// forward and two backward, with their LDS reads and writes: 46 of 64 us at
+// 1024 x 1500, the rest the loads and stores of the columns (32 bytes of a row
+// per workgroup; groups of modes that share lines go to one XCD, 23 us against 32
+// without).  The chains in global memory waited for each step's loads and
+// divided: 390 us at 256 x 511 and 1113 us at 1024 x 1500, now 28 and 69 (HIP
+// events, about 5 us of them the events').  A chunked solve would be 3 times
+// faster again, but rounds differently: in mixed precision that moves the shear
+// stress, formed in FP32 from the velocity, by 5e-9.
+__global__ void k_tdm_factors(double* __restrict__ v, double* __restrict__ q1, double* __restrict__ cl, int nx, int ny,
+                              const double* __restrict__ evals, double l, double u) {
+  const int mo = blockIdx.x * blockDim.x + threadIdx.x;
+  if (mo >= nx) return;
+  const double c = -l - u + evals[mo];
+  const int n = ny, N = ny - 1;
+#define V(r) v[(size_t)(r) * nx + mo]
+#define Q1(r) q1[(size_t)(r) * nx + mo]
+  V(0) = 0.;  // (row 0 divides by c)
+  double vp = u / c;
+  double x = -l / c;
+  Q1(0) = x;
+  for (int r = 1; r < N - 1; r++) {
+    const double val = 1. / (c - l * vp);
+    vp = val * u;
+    x = val * (((r == n - 2) ? -u : 0.) - l * x);
+    V(r) = val;
+    Q1(r) = x;
+  }
+  {
+    // (an inverse of 0 marks the reference's singular pivot: its row is 0)
+    const double val = c - l * vp;
+    const bool ok = fabs(val) > DBL_EPSILON;
+    V(N - 1) = ok ? 1. / val : 0.;
+    x = ok ? 1. / val * (((N - 1 == n - 2) ? -u : 0.) - l * x) : 0.;
+    Q1(N - 1) = x;
+  }
+  const double v0 = u / c, last = x;
+  for (int r = N - 2; r >= 0; r--) {
+    x = Q1(r) - (r ? V(r) * u : v0) * x;
+    Q1(r) = x;
+  }
+  cl[mo] = c + u * x + l * last;
+#undef V
+#undef Q1
+}
+
+template <int MW>
+__device__ __forceinline__ void tdm_column_body(double* __restrict__ q, const double* __restrict__ v,
+                                                const double* __restrict__ q1, const double* __restrict__ cl, int nx,
+                                                int ny, const double* __restrict__ evals, double l, double u, int pin,
+                                                int m0, double2* lds) {
+  constexpr int kB = kColumnBatch, T = 256;
+  const int N = ny - 1, n = ny * MW, t = (int)threadIdx.x;
+  // {right-hand side, inverse pivot} of row r and mode m0 + m at col[r MW + m],
+  // with kColumnPad rows at both ends, which the batches that run past the
+  // column read and do not use
+  double2* col = lds + kColumnPad * MW;
+#pragma unroll 8
+  for (int e = t; e < n; e += T) {
+    const size_t o = (size_t)(e / MW) * nx + min(m0 + e % MW, nx - 1);
+    col[e] = make_double2(q[o], v[e < n - MW ? o : o - nx]);  // (the last row takes no pivot)
+  }
+  __syncthreads();
+  if (t < MW) {
+    const int mo = min(m0 + t, nx - 1);
+    const double c = -l - u + evals[mo], v0 = u / c;
+    // Full batches of rows without a test, their rows read two batches ahead of
+    // the chain (three register sets in turn: an LDS read takes longer than the
+    // chain of one batch), then guarded batches.
+    double ax[kB], aw[kB], bx[kB], bw[kB], cx[kB], cw[kB];
+    auto load = [](double* x, double* w, const double2* s, int step) {
+#pragma unroll
+      for (int k = 0; k < kB; k++) {
+        const double2 d = s[k * step];
+        x[k] = d.x;
+        w[k] = d.y;
+      }
+    };
+    double y = col[t].x / c;
+    col[t].x = y;
+    {
+      double2* p = col + MW + t;
+      auto chain = [&](const double* x, const double* w, double2* s, int rows) {
+#pragma unroll
+        for (int k = 0; k < kB; k++)
+          if (k < rows) {
+            y = w[k] * (x[k] - l * y);
+            s[k * MW].x = y;
+          }
+      };
+      int left = N - 2;  // rows 1 .. N - 2
+      load(ax, aw, p, MW);
+      load(bx, bw, p + kB * MW, MW);
+      for (; left >= 3 * kB; left -= 3 * kB, p += 3 * kB * MW) {
+        load(cx, cw, p + 2 * kB * MW, MW);
+        chain(ax, aw, p, kB);
+        load(ax, aw, p + 3 * kB * MW, MW);
+        chain(bx, bw, p + kB * MW, kB);
+        load(bx, bw, p + 4 * kB * MW, MW);
+        chain(cx, cw, p + 2 * kB * MW, kB);
+      }
+      for (; left > 0; left -= kB, p += kB * MW) {
+        load(ax, aw, p, MW);
+        chain(ax, aw, p, left);
+      }
+      // row N - 1 (0 where its pivot is singular)
+      double2* e = col + (N - 1) * MW + t;
+      y = e->y == 0. ? 0. : e->y * (e->x - l * y);
+      e->x = y;
+    }
+    {
+      const double last = y;
+      double2* p = col + (N - 2) * MW + t;
+      auto chain = [&](const double* x, const double* w, double2* s, int rows) {
+#pragma unroll
+        for (int k = 0; k < kB; k++)
+          if (k < rows) {
+            y = x[k] - w[k] * u * y;
+            s[-k * MW].x = y;
+          }
+      };
+      int left = N - 2;  // rows N - 2 .. 1
+      load(ax, aw, p, -MW);
+      load(bx, bw, p - kB * MW, -MW);
+      for (; left >= 3 * kB; left -= 3 * kB, p -= 3 * kB * MW) {
+        load(cx, cw, p - 2 * kB * MW, -MW);
+        chain(ax, aw, p, kB);
+        load(ax, aw, p - 3 * kB * MW, -MW);
+        chain(bx, bw, p - kB * MW, kB);
+        load(bx, bw, p - 4 * kB * MW, -MW);
+        chain(cx, cw, p - 2 * kB * MW, kB);
+      }
+      for (; left > 0; left -= kB, p -= kB * MW) {
+        load(ax, aw, p, -MW);
+        chain(ax, aw, p, left);
+      }
+      y = col[t].x - v0 * y;
+      col[t].x = y;
+      const double num = col[N * MW + t].x - u * y - l * last;
+      const double den = cl[mo];
+      col[N * MW + t].x = ((pin && mo == 0) || fabs(den) < DBL_EPSILON) ? 0. : num / den;
+    }
+  }
+  __syncthreads();
+#pragma unroll 8
+  for (int e = t; e < n; e += T) {
+    const int m = e % MW;
+    if (m0 + m >= nx) continue;
+    const size_t o = (size_t)(e / MW) * nx + m0 + m;
+    q[o] = e < n - MW ? col[e].x + col[n - MW + m].x * q1[o] : col[e].x;
+  }
+}
+
+template <int MW>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) void k_tdm_columns(double* __restrict__ q, const double* __restrict__ v,
+                                                     const double* __restrict__ q1, const double* __restrict__ cl,
+                                                     int nx, int ny, const double* __restrict__ evals, double l,
+                                                     double u, int pin) {
+  extern __shared__ double2 col[];
+  tdm_column_body<MW>(q, v, q1, cl, nx, ny, evals, l, u, pin, xcd_group((int)blockIdx.x, (int)gridDim.x) * MW, col);
+}
+
+// scratch, or the tables, of the sequential solve; synchronous, on the first
+// (eager) pass that takes it
+static int sequential_setup(PoissonPlan* p, double l) {
+  if (p->cl) return 0;
+  const size_t cells = (size_t)p->nx * p->ny;
+  if (!p->v) SBFS_HIP(hipMalloc(&p->v, sizeof(double) * cells));
+  if (!p->q1) SBFS_HIP(hipMalloc(&p->q1, sizeof(double) * cells));
+  double* cl = nullptr;
+  SBFS_HIP(hipMalloc(&cl, sizeof(double) * p->nx));
+  if (tdm_columns(p->ny)) {
+    hipLaunchKernelGGL(k_tdm_factors, dim3(cdiv(p->nx, 64)), dim3(64), 0, stream(), p->v, p->q1, cl, p->nx, p->ny,
+                       p->evals, l, l);
+    if (check_launch("poisson: tridiagonal factors")) {
+      (void)hipFree(cl);
+      return 1;
+    }
+  }
+  p->cl = cl;
+  return 0;
+}
+
+static int sequential_solve(PoissonPlan* p, double l, int pin) {
+  if (sequential_setup(p, l)) return 1;
+  const int nx = p->nx, ny = p->ny, mw = tdm_columns(ny);
+  const size_t lds = tdm_column_lds(ny, mw);
+#define SBFS_COLUMNS(MW)                                                                                            SBFS_TIMED("k_tdm_columns", hipLaunchKernelGGL(k_tdm_columns<MW>, dim3(cdiv(nx, MW)), dim3(256), lds, stream(),                                                  p->buf, (const double*)p->v, (const double*)p->q1,                                                                (const double*)p->cl, nx, ny, (const double*)p->evals, l, l, pin))
+  if (mw == 4) SBFS_COLUMNS(4);
+  else if (mw == 2) SBFS_COLUMNS(2);
+  else if (mw == 1) SBFS_COLUMNS(1);
+#undef SBFS_COLUMNS
+  else
+    SBFS_TIMED("k_tdm_sequential", hipLaunchKernelGGL(k_tdm_sequential, dim3(cdiv(nx, 64)), dim3(64), 0, stream(),
+                                                      p->buf, p->v, p->q1, nx, ny, p->evals, l, l, pin));
+  return check_launch("poisson: tridiagonal");
+}
+
 // ensembles: one map entry (case, group of rows or of 64 modes) per
 // workgroup; the row transforms switch on the case's transform length,
 // which is uniform over the wavefront
@@ -652,6 +854,21 @@ __global__ void k_tdm_sequential_batch(const RowArgs* __restrict__ tab, const ui
   const uint2 mp = map[blockIdx.x];
   const RowArgs& a = tab[mp.x];
   tdm_sequential_body(a.buf, a.v, a.q1, a.nx, a.ny, a.evals, a.l, a.l, a.pin, (int)mp.y * 64 + threadIdx.x);
+}
+
+// one map entry (case, group of tdm_columns(ny) modes) per workgroup
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) void k_tdm_columns_batch(const RowArgs* __restrict__ tab,
+                                                           const uint2* __restrict__ map) {
+  extern __shared__ double2 col[];
+  const uint2 mp = map[blockIdx.x];
+  const RowArgs& a = tab[mp.x];
+  switch (tdm_columns(a.ny)) {
+#define SBFS_COLUMN_CASE(MW)   case MW: tdm_column_body<MW>(a.buf, a.v, a.q1, a.cl, a.nx, a.ny, a.evals, a.l, a.l, a.pin, (int)mp.y * MW, col); break
+    SBFS_COLUMN_CASE(4);
+    SBFS_COLUMN_CASE(2);
+    SBFS_COLUMN_CASE(1);
+#undef SBFS_COLUMN_CASE
+  }
 }
 
 __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2))) void k_dct3_psi_batch(
@@ -681,10 +898,7 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2))) void k
 // ---------------------------------------------------------------------------
 static int plan_build(PoissonPlan* p, const domain_t* d) {
   const int nx = p->nx, ny = p->ny, m = p->m;
-  const size_t cells = (size_t)nx * ny;
-  SBFS_HIP(hipMalloc(&p->buf, sizeof(double) * cells));
-  SBFS_HIP(hipMalloc(&p->v, sizeof(double) * cells));
-  SBFS_HIP(hipMalloc(&p->q1, sizeof(double) * cells));
+  SBFS_HIP(hipMalloc(&p->buf, sizeof(double) * (size_t)nx * ny));
   SBFS_HIP(hipMalloc(&p->evals, sizeof(double) * nx));
   SBFS_HIP(hipMalloc(&p->tw, sizeof(double2) * (m > 0 ? m : 1)));
   SBFS_HIP(hipMalloc(&p->t1, sizeof(double2) * (m + 1)));
@@ -776,10 +990,7 @@ static int poisson_tail(const domain_t* d, PoissonPlan* p, fluid_t* f) {
     const int K = L - 1;
     src = ModeSrc{p->buf, p->X, p->ptab + (size_t)2 * K * nx, p->ptab + (size_t)3 * K * nx, nx, L, p->P};
   } else {
-    SBFS_TIMED("k_tdm_sequential",
-               hipLaunchKernelGGL(k_tdm_sequential, dim3(cdiv(nx, 64)), dim3(64), 0, stream(),
-                                  p->buf, p->v, p->q1, nx, ny, p->evals, l, l, pin));
-    if (check_launch("poisson: tridiagonal")) return 1;
+    if (sequential_solve(p, l, pin)) return 1;
   }
   double* psi = (double*)f->psi[1].data;
   SBFS_REQUIRE(((uintptr_t)psi & 15) == 0, "poisson: psi[1] must be 16-byte aligned (hipMalloc'ed)");
@@ -833,8 +1044,6 @@ int poisson_row_args(const domain_t* d, DomainCtx* c, double* psi, RowArgs* a) {
   if (!p->rhs) SBFS_HIP(hipMalloc(&p->rhs, sizeof(double) * (size_t)p->nx * p->ny));
   a->rhs = p->rhs;
   a->buf = p->buf;
-  a->v = p->v;
-  a->q1 = p->q1;
   SBFS_REQUIRE(((uintptr_t)psi & 15) == 0, "poisson: psi[1] must be 16-byte aligned (hipMalloc'ed)");
   a->psi = psi;
   a->evals = p->evals;
@@ -862,7 +1071,12 @@ int poisson_row_args(const domain_t* d, DomainCtx* c, double* psi, RowArgs* a) {
     a->gfl = p->gfl;
     a->X = p->X;
     a->pa = p->a;
+  } else if (sequential_setup(p, a->l)) {
+    return 1;
   }
+  a->v = p->v;
+  a->q1 = p->q1;
+  a->cl = p->cl;
   return 0;
 }
 

@@ -18,8 +18,11 @@ struct PoissonPlan {
   double lx = 0.;
   double* buf = nullptr;     // nx * ny, modes r[j][m]
   double* rhs = nullptr;     // nx * ny, right-hand side rows (marching path)
-  double* v = nullptr;       // nx * ny, sequential-solver factors
-  double* q1 = nullptr;      // nx * ny, sequential-solver spike
+  // sequential solver (allocated when it is first used): with columns in LDS
+  // (tdm_columns) the tables that do not depend on the data, else scratch
+  double* v = nullptr;       // nx * ny: inverse pivots / factors
+  double* q1 = nullptr;      // nx * ny: solution of the corner spike
+  double* cl = nullptr;      // nx: the closure's denominator
   double* evals = nullptr;   // nx
   double2* tw = nullptr;     // m      FFT twiddles e^{-2 pi i e/m}
   double2* t1 = nullptr;     // m + 1  e^{-2 pi i k/n}
@@ -39,6 +42,7 @@ struct RowArgs {
   double* buf;        // modes
   double* v;
   double* q1;
+  const double* cl;
   double* psi;        // psi[1] of the stage
   const double* evals;
   const double2* tw;
@@ -57,6 +61,21 @@ struct RowArgs {
 int poisson_row_args(const domain_t* d, DomainCtx* c, double* psi, RowArgs* a);
 __global__ void k_dct2_rows_batch(const RowArgs* tab, const uint2* map);
 __global__ void k_tdm_sequential_batch(const RowArgs* tab, const uint2* map);
+__global__ void k_tdm_columns_batch(const RowArgs* tab, const uint2* map);
+// The sequential solve with whole columns in LDS: modes per workgroup (0: the
+// columns do not fit, k_tdm_sequential) and its LDS bytes, the right-hand side
+// and the inverse pivots of each.
+constexpr size_t kColumnLds = 160 << 10;
+constexpr int kColumnBatch = 8, kColumnPad = 2 * kColumnBatch;  // rows read together, and past a column's ends
+__host__ __device__ inline size_t tdm_column_lds(int ny, int modes) {
+  return sizeof(double2) * (size_t)(ny + 2 * kColumnPad) * modes;
+}
+__host__ __device__ inline int tdm_columns(int ny) {
+  return tdm_column_lds(ny, 4) <= kColumnLds ? 4
+         : tdm_column_lds(ny, 2) <= kColumnLds ? 2
+         : tdm_column_lds(ny, 1) <= kColumnLds ? 1
+                                               : 0;
+}
 __global__ void k_dct3_psi_batch(const RowArgs* tab, const uint2* map);
 __global__ void k_part_reduce_batch(const RowArgs* tab, const uint2* map);
 __global__ void k_part_conv_batch(const RowArgs* tab, const uint2* map);
