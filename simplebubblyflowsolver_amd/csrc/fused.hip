@@ -19,6 +19,8 @@
 #include <cstdint>
 #include <cstdlib>
 #include <cstring>
+#include <mutex>
+#include <utility>
 #include <vector>
 
 #include "decide_dt.h"
@@ -207,6 +209,7 @@ struct FusedScratch {
   double* ux2 = nullptr;  // predicted velocity of stage 1 (folded projection)
   double* uy2 = nullptr;
   double* p = nullptr;    // pressure written by a stage kernel with the folded projection
+  // learned curvature only (allocated when it is first used):
   float* kappa = nullptr;  // learned curvature of a stage's input vof (interior cells)
   unsigned* klist[3] = {};  // its listed cells (count first), one list per stage
   int klast = -1;            // the list of the last launch (-1: none since the fill)
@@ -216,61 +219,142 @@ struct FusedScratch {
   unsigned* order = nullptr;
   int units = 0;
 };
-static FusedScratch g_scr;
-
-static int scratch(const domain_t* d, const interface_t* s, const fluid_t* f) {
-  if (g_scr.nx == d->mysizes[0] && g_scr.ny == d->mysizes[1]) return 0;
-  (void)hipStreamSynchronize(stream());
-  graph_epoch_bump();
-  for (double* q : {g_scr.vof, g_scr.ux, g_scr.uy, g_scr.ux2, g_scr.uy2, g_scr.p}) (void)hipFree(q);
-  (void)hipFree(g_scr.kappa);
-  for (unsigned* l : g_scr.klist) (void)hipFree(l);
-  (void)hipFree(g_scr.cut);
-  (void)hipFree(g_scr.weight);
-  (void)hipFree(g_scr.order);
-  g_scr = FusedScratch();
-  const std::pair<double**, size_t> bufs[] = {{&g_scr.vof, s->vof.datasize}, {&g_scr.ux, f->ux.datasize},
-                                              {&g_scr.uy, f->uy.datasize},   {&g_scr.ux2, f->ux.datasize},
-                                              {&g_scr.uy2, f->uy.datasize},  {&g_scr.p, f->p.datasize}};
-  for (const auto& b : bufs) {
-    SBFS_HIP(hipMalloc(b.first, b.second));
-    SBFS_HIP(hipMemsetAsync(*b.first, 0, b.second, stream()));
-  }
-  const size_t cells = d->mysizes[0] * d->mysizes[1];
-  SBFS_HIP(hipMalloc(&g_scr.kappa, sizeof(float) * cells));
-  for (unsigned*& l : g_scr.klist) SBFS_HIP(hipMalloc(&l, sizeof(unsigned) * (cells + 1)));
-  if (curv_field_init(g_scr.kappa, g_scr.klist, 3, (long)cells, stream())) return 1;
-  g_scr.klast = -1;
-  SBFS_HIP(hipMalloc(&g_scr.cut, sizeof(unsigned long long) * d->mysizes[1] * march_strips((int)d->mysizes[0])));
-  g_scr.nx = d->mysizes[0];
-  g_scr.ny = d->mysizes[1];
-  return 0;
-}
-
-// weight and order buffers for n units (zero weights at first: any order)
-static int order_buffers(int n) {
-  if (g_scr.units >= n) return 0;
-  (void)hipStreamSynchronize(stream());
-  graph_epoch_bump();
-  (void)hipFree(g_scr.weight);
-  (void)hipFree(g_scr.order);
-  g_scr.weight = g_scr.order = nullptr;
-  g_scr.units = 0;
-  SBFS_HIP(hipMalloc(&g_scr.weight, sizeof(unsigned) * (size_t)n));
-  SBFS_HIP(hipMalloc(&g_scr.order, sizeof(unsigned) * (size_t)n));
-  SBFS_HIP(hipMemsetAsync(g_scr.weight, 0, sizeof(unsigned) * (size_t)n, stream()));
-  g_scr.units = n;
-  return 0;
-}
 
 struct CoefTables {
-  const DomainCtx* ctx = nullptr;
-  uint64_t hash = 0;
   double re = 0.;
   double* buf = nullptr;
   Coef cf{};
 };
-static CoefTables g_coef;
+
+// A step graph's key, and the state it leaves
+struct StepKey {
+  std::vector<uint64_t> v;
+  bool operator==(const StepKey& o) const { return v == o.v; }
+};
+
+constexpr int kStateArrays = 17;
+struct StepGraph {
+  StepKey key;
+  hipGraphExec_t exec = nullptr;
+  // state pointers after the step, then the scratch vof and pressure, which
+  // a step swaps with the state's (the pressure once per step)
+  void* after[kStateArrays + 2] = {};
+  uint64_t last_use = 0;
+};
+
+// Everything the fused step keeps from one step of a domain to the next, owned
+// by the domain's context: scratch, coefficient tables, the stage kernels'
+// arguments in device memory and the captured steps.  One set per process made
+// every step of a program that advances several cases in turn rebuild the
+// tables (a synchronisation, a hipFree and a hipMalloc) and launch eagerly, the
+// two graphs having been captured for other cases: 294 us per step for three
+// 64 x 128 bubbles in turn against 233 for one, 1946 against 1544 for three
+// 2048 x 4096 swarms.  A step has two pointer states, so four graphs serve
+// two fluids on one domain.
+struct ArgsSlot {
+  MarchArgs host;
+  MarchArgs* dev;
+};
+constexpr int kStepGraphs = 4;
+constexpr size_t kMaxArgSlots = 64;
+struct FusedState {
+  FusedScratch scr;
+  CoefTables coef;
+  std::vector<ArgsSlot> args;
+  MarchArgs* args_dev = nullptr;  // kMaxArgSlots
+  StepGraph graph[kStepGraphs];
+  StepKey seen[kStepGraphs];
+  uint64_t clock = 0;
+};
+
+static void scratch_free(FusedScratch& s) {
+  for (double* q : {s.vof, s.ux, s.uy, s.ux2, s.uy2, s.p}) (void)hipFree(q);
+  (void)hipFree(s.kappa);
+  for (unsigned* l : s.klist) (void)hipFree(l);
+  (void)hipFree(s.cut);
+  (void)hipFree(s.weight);
+  (void)hipFree(s.order);
+  s = FusedScratch();
+}
+
+// The scratch of the last domain given back, for the next one of its size: a
+// program that closes a case and opens another allocates no scratch.  One set
+// at most.
+static std::mutex g_spare_mutex;
+static FusedScratch g_spare;
+
+// (the caller has synchronised the stream)
+void fused_destroy(FusedState* s) {
+  if (!s) return;
+  for (StepGraph& g : s->graph)
+    if (g.exec) (void)hipGraphExecDestroy(g.exec);
+  (void)hipFree(s->coef.buf);
+  (void)hipFree(s->args_dev);
+  if (s->scr.vof) {
+    std::lock_guard<std::mutex> lock(g_spare_mutex);
+    scratch_free(g_spare);
+    g_spare = s->scr;
+  }
+  delete s;
+}
+
+static int scratch(DomainCtx* c, const interface_t* s, const fluid_t* f, bool learned) {
+  FusedScratch& scr = c->fused->scr;
+  const size_t cells = c->nx * c->ny;
+  if (!scr.vof) {
+    {
+      std::lock_guard<std::mutex> lock(g_spare_mutex);
+      if (g_spare.vof && g_spare.nx == c->nx && g_spare.ny == c->ny) {
+        scr = g_spare;
+        g_spare = FusedScratch();
+      }
+    }
+    if (!scr.vof) {
+      const std::pair<double**, size_t> bufs[] = {{&scr.ux, f->ux.datasize},   {&scr.uy, f->uy.datasize},
+                                                  {&scr.ux2, f->ux.datasize},  {&scr.uy2, f->uy.datasize},
+                                                  {&scr.p, f->p.datasize},     {&scr.vof, s->vof.datasize}};
+      // (the vof last: it marks the set as whole)
+      for (const auto& b : bufs) {
+        (void)hipFree(*b.first);
+        *b.first = nullptr;
+        double* q = nullptr;
+        SBFS_HIP(hipMalloc(&q, b.second));
+        const hipError_t e = hipMemsetAsync(q, 0, b.second, stream());
+        if (e != hipSuccess) (void)hipFree(q);
+        SBFS_HIP(e);
+        *b.first = q;
+      }
+      scr.nx = c->nx;
+      scr.ny = c->ny;
+    }
+  }
+  if (learned && !scr.cut) {
+    if (!scr.kappa) SBFS_HIP(hipMalloc(&scr.kappa, sizeof(float) * cells));
+    for (unsigned*& l : scr.klist)
+      if (!l) SBFS_HIP(hipMalloc(&l, sizeof(unsigned) * (cells + 1)));
+    if (curv_field_init(scr.kappa, scr.klist, 3, (long)cells, stream())) return 1;
+    scr.klast = -1;
+    SBFS_HIP(hipMalloc(&scr.cut, sizeof(unsigned long long) * c->ny * march_strips((int)c->nx)));
+  }
+  return 0;
+}
+
+// weight and order buffers for n units (zero weights at first: any order)
+static int order_buffers(DomainCtx* c, int n) {
+  FusedScratch& scr = c->fused->scr;
+  if (scr.units >= n) return 0;
+  (void)hipStreamSynchronize(stream());
+  c->epoch++;
+  (void)hipFree(scr.weight);
+  (void)hipFree(scr.order);
+  scr.weight = scr.order = nullptr;
+  scr.units = 0;
+  SBFS_HIP(hipMalloc(&scr.weight, sizeof(unsigned) * (size_t)n));
+  SBFS_HIP(hipMalloc(&scr.order, sizeof(unsigned) * (size_t)n));
+  SBFS_HIP(hipMemsetAsync(scr.weight, 0, sizeof(unsigned) * (size_t)n, stream()));
+  scr.units = n;
+  return 0;
+}
 
 // the 14 per-column quotient tables of one domain and Re in a new device
 // buffer (*buf, owned by the caller)
@@ -324,23 +408,19 @@ int coef_build(const domain_t* d, double Re, double** buf, Coef* out) {
   return 0;
 }
 
-static int coef_tables(const domain_t* d, const DomainCtx* c, double Re, Coef* out) {
-  if (g_coef.ctx == c && g_coef.hash == c->hash && g_coef.re == Re && g_coef.buf) {
-    *out = g_coef.cf;
-    return 0;
+static int coef_tables(const domain_t* d, DomainCtx* c, double Re, Coef* out) {
+  CoefTables& t = c->fused->coef;
+  if (!t.buf || t.re != Re) {
+    (void)hipStreamSynchronize(stream());
+    c->epoch++;
+    (void)hipFree(t.buf);
+    t.buf = nullptr;
+    if (coef_build(d, Re, &t.buf, &t.cf)) return 1;
+    t.re = Re;
   }
-  (void)hipStreamSynchronize(stream());
-  graph_epoch_bump();
-  (void)hipFree(g_coef.buf);
-  g_coef.buf = nullptr;
-  if (coef_build(d, Re, &g_coef.buf, &g_coef.cf)) return 1;
-  g_coef.ctx = c;
-  g_coef.hash = c->hash;
-  g_coef.re = Re;
-  *out = g_coef.cf;
+  *out = t.cf;
   return 0;
 }
-
 
 int poisson_transform_fused(const domain_t* d, DomainCtx* c, fluid_t* f, double** rhs);  // poisson.hip
 
@@ -529,52 +609,39 @@ static void fill_post(const DomainCtx* c, const fluid_t* fluid, const interface_
 
 // The stage kernels' arguments in device memory (the kernels read them
 // through a pointer, march.hip).  A step configuration builds the same
-// arguments at every step, so they sit in a small cache keyed by their
-// bytes: the eager first pass of a configuration uploads them (a
-// synchronous copy, allowed there), and the graph captured on its second
-// pass finds the same bytes and records only the pointer.  The cache is
-// emptied when the graph epoch moves (buffers were freed) or when it fills.
-struct ArgsSlot {
-  MarchArgs host;
-  MarchArgs* dev;
-};
-static std::vector<ArgsSlot> g_args;
-static uint64_t g_args_epoch = 0;
-constexpr size_t kMaxArgSlots = 64;
-
-static void args_clear() {
-  (void)hipStreamSynchronize(stream());
-  for (ArgsSlot& s : g_args) (void)hipFree(s.dev);
-  g_args.clear();
+// arguments at every step, so they sit in a small cache of the domain keyed by
+// their bytes: the eager first pass of a configuration stores them with a
+// one-workgroup kernel (no host synchronisation), and the graph captured on its
+// second pass finds the same bytes and records only the pointer.
+__global__ void k_store_args(MarchArgs m, MarchArgs* __restrict__ out) {
+  static_assert(sizeof(MarchArgs) % 8 == 0, "copied by 8-byte words");
+  const unsigned long long* s = (const unsigned long long*)&m;
+  unsigned long long* d = (unsigned long long*)out;
+  for (int k = threadIdx.x; k < (int)(sizeof(MarchArgs) / 8); k += blockDim.x) d[k] = s[k];
 }
 
-static int device_args(const MarchArgs& m, const MarchArgs** out) {
-  if (g_args_epoch != graph_epoch()) {
-    args_clear();
-    g_args_epoch = graph_epoch();
-  }
-  for (const ArgsSlot& s : g_args)
-    if (memcmp(&s.host, &m, sizeof(m)) == 0) {
-      *out = s.dev;
+static int device_args(DomainCtx* c, const MarchArgs& m, const MarchArgs** out) {
+  FusedState& s = *c->fused;
+  for (const ArgsSlot& a : s.args)
+    if (memcmp(&a.host, &m, sizeof(m)) == 0) {
+      *out = a.dev;
       return 0;
     }
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   SBFS_HIP(hipStreamIsCapturing(stream(), &cs));
   SBFS_REQUIRE(cs == hipStreamCaptureStatusNone,
                "integrate: stage arguments of a captured step were not prepared by its eager pass");
-  if (g_args.size() >= kMaxArgSlots) {
-    // captured graphs may hold the old pointers: move the epoch so that
-    // none of them replays
-    args_clear();
-    graph_epoch_bump();
-    g_args_epoch = graph_epoch();
+  if (!s.args_dev) SBFS_HIP(hipMalloc(&s.args_dev, sizeof(MarchArgs) * kMaxArgSlots));
+  if (s.args.size() >= kMaxArgSlots) {
+    // captured graphs hold pointers to these slots: move the epoch so that
+    // none of them replays (queued steps read them before the stores below)
+    s.args.clear();
+    c->epoch++;
   }
-  MarchArgs* d = nullptr;
-  SBFS_HIP(hipMalloc(&d, sizeof(MarchArgs)));
-  const hipError_t e = hipMemcpy(d, &m, sizeof(MarchArgs), hipMemcpyHostToDevice);
-  if (e != hipSuccess) (void)hipFree(d);
-  SBFS_HIP(e);
-  g_args.push_back({m, d});
+  MarchArgs* d = s.args_dev + s.args.size();
+  hipLaunchKernelGGL(k_store_args, dim3(1), dim3(64), 0, stream(), m, d);
+  if (check_launch("integrate: stage arguments")) return 1;
+  s.args.push_back({m, d});
   *out = d;
   return 0;
 }
@@ -585,6 +652,7 @@ static int device_args(const MarchArgs& m, const MarchArgs** out) {
 // synchronisation, so the sequence can be captured into a graph.
 static int fused_body(const domain_t* domain, DomainCtx* c, fluid_t* fluid, interface_t* interface,
                       const Coef& cf, double* rhs, int band, double learned_h) {
+  FusedScratch& scr = c->fused->scr;
   const int nx = (int)c->nx, ny = (int)c->ny;
   // learned curvature of each stage's input vof: on the side stream, forked
   // after the kernel that wrote that vof and joined before the stage kernel
@@ -596,20 +664,20 @@ static int fused_body(const domain_t* domain, DomainCtx* c, fluid_t* fluid, inte
   // (stages 1 and 2 list their cells from the previous stage kernel's
   // bitmask of the vof it wrote; stage 0 from the state's vof, which the
   // caller may have changed since the last step)
-  auto cut_of = [](int k) -> const unsigned long long* { return k > 0 ? g_scr.cut : nullptr; };
+  auto cut_of = [&scr](int k) -> const unsigned long long* { return k > 0 ? scr.cut : nullptr; };
   // stage k lists into list k; the launch before it wrote list klast, and
   // the launch after it writes list (k + 1) % 3
   auto curv_launch = [&](int k, const double* vof, hipStream_t st) -> int {
-    if (g_scr.klast == k) {
+    if (scr.klast == k) {
       // only after a step that stopped part way: start the field afresh
-      if (curv_field_init(g_scr.kappa, g_scr.klist, 3, (long)nx * ny, st)) return 1;
-      g_scr.klast = -1;
+      if (curv_field_init(scr.kappa, scr.klist, 3, (long)nx * ny, st)) return 1;
+      scr.klast = -1;
     }
-    const unsigned* prev = g_scr.klast >= 0 ? g_scr.klist[g_scr.klast] : nullptr;
-    if (curv_mlp_launch(vof, cut_of(k), g_scr.kappa, g_scr.klist[k], prev, g_scr.klist[(k + 1) % 3], nx, ny,
+    const unsigned* prev = scr.klast >= 0 ? scr.klist[scr.klast] : nullptr;
+    if (curv_mlp_launch(vof, cut_of(k), scr.kappa, scr.klist[k], prev, scr.klist[(k + 1) % 3], nx, ny,
                         learned_h, st))
       return 1;
-    g_scr.klast = k;
+    scr.klast = k;
     return 0;
   };
   auto fork_curv = [&](int k, const double* vof) -> int {
@@ -631,16 +699,16 @@ static int fused_body(const domain_t* domain, DomainCtx* c, fluid_t* fluid, inte
   const bool ordered = march_ordered(mixed);
   const int units = march_units(nx, ny, band);
   if (ordered) {
-    SBFS_REQUIRE(g_scr.units >= units, "integrate: no dispatch-order buffers for %d units", units);
+    SBFS_REQUIRE(scr.units >= units, "integrate: no dispatch-order buffers for %d units", units);
     SBFS_TIMED("k_march_order", hipLaunchKernelGGL(k_march_order, dim3(1), dim3(1024), 0, stream(),
-                                                   (const unsigned*)g_scr.weight, g_scr.order, units,
+                                                   (const unsigned*)scr.weight, scr.order, units,
                                                    march_max_weight(band)));
     if (check_launch("integrate: k_march_order")) return 1;
   }
   // predicted velocity of each stage: with the fold, stage 1 writes the
   // second pair while it reads the first
-  double* const us[3] = {g_scr.ux, fold ? g_scr.ux2 : g_scr.ux, g_scr.ux};
-  double* const vs[3] = {g_scr.uy, fold ? g_scr.uy2 : g_scr.uy, g_scr.uy};
+  double* const us[3] = {scr.ux, fold ? scr.ux2 : scr.ux, scr.ux};
+  double* const vs[3] = {scr.uy, fold ? scr.uy2 : scr.uy, scr.uy};
   for (int k = 0; k < 3; k++) {
     const bool corr = fold && k > 0;  // this stage applies stage k-1's projection
     if (k != 0) {
@@ -651,24 +719,24 @@ static int fused_body(const domain_t* domain, DomainCtx* c, fluid_t* fluid, inte
     {
       MarchArgs m;
       memset(&m, 0, sizeof(m));  // padding too: the arguments are compared bytewise
-      fill_march(domain, c, fluid, interface, cf, rhs, band, k, corr, us, vs, g_scr.vof, g_scr.p, dtp, m);
+      fill_march(domain, c, fluid, interface, cf, rhs, band, k, corr, us, vs, scr.vof, scr.p, dtp, m);
       if (learned) {
         if (overlap) {
           SBFS_HIP(hipStreamWaitEvent(stream(), join_event(k), 0));
         } else if (curv_launch(k, D(interface->vof), stream())) {
           return 1;
         }
-        m.kappa = g_scr.kappa;
-        m.kappa_n = g_scr.klist[k];
-        if (k < 2) m.cut = g_scr.cut;
+        m.kappa = scr.kappa;
+        m.kappa_n = scr.klist[k];
+        if (k < 2) m.cut = scr.cut;
       }
       if (ordered) {
-        m.order = g_scr.order;
-        m.weight = g_scr.weight;
+        m.order = scr.order;
+        m.weight = scr.weight;
       }
       const dim3 grid = ordered ? dim3(units) : dim3(cdiv(nx, kStrip), cdiv(ny, band)), block(64);
       const MarchArgs* ma = nullptr;
-      if (device_args(m, &ma)) return 1;
+      if (device_args(c, m, &ma)) return 1;
       if (mixed && corr)
         SBFS_TIMED("k_march_mixed_corr", hipLaunchKernelGGL(k_march_mixed_corr, grid, block, 0, stream(), ma));
       else if (mixed)
@@ -681,15 +749,15 @@ static int fused_body(const domain_t* domain, DomainCtx* c, fluid_t* fluid, inte
       if (corr && k == 2) {
         // the stage kernel wrote the pressure after stage 1's update
         double* t = (double*)fluid->p.data;
-        fluid->p.data = g_scr.p;
-        g_scr.p = t;
+        fluid->p.data = scr.p;
+        scr.p = t;
       }
     }
     {
       // the new vof becomes the state; the old one is the next scratch
       void* t = interface->vof.data;
-      interface->vof.data = g_scr.vof;
-      g_scr.vof = (double*)t;
+      interface->vof.data = scr.vof;
+      scr.vof = (double*)t;
     }
     // the next stage's curvature from the new vof, beside this stage's
     // Poisson solve (the stage kernel that read kappa has been launched)
@@ -726,11 +794,6 @@ static int fused_body(const domain_t* domain, DomainCtx* c, fluid_t* fluid, inte
 // synchronises nothing.  Profiling (per-launch events) and SBFS_GRAPH=0
 // keep the eager path.
 // ---------------------------------------------------------------------------
-struct StepKey {
-  std::vector<uint64_t> v;
-  bool operator==(const StepKey& o) const { return v == o.v; }
-};
-
 static void key_add(StepKey& k, const void* p) { k.v.push_back((uint64_t)(uintptr_t)p); }
 static void key_add(StepKey& k, double x) {
   uint64_t u;
@@ -744,20 +807,21 @@ static array_t* state_arrays(fluid_t* f, interface_t* s, int k) {
                   &f->srcuy[1], &f->srcuy[2], &s->vof, &s->src[0], &s->src[1]};
   return k < 17 ? a[k] : nullptr;
 }
-constexpr int kStateArrays = 17;
 
 static StepKey step_key(const DomainCtx* c, fluid_t* f, interface_t* s, const Coef& cf, double* rhs,
                         int band) {
+  const FusedScratch& scr = c->fused->scr;
   StepKey k;
+  k.v.reserve(64);
   key_add(k, c);
   k.v.push_back(c->hash);
   for (int n = 0; n < kStateArrays; n++) key_add(k, state_arrays(f, s, n)->data);
-  key_add(k, g_scr.vof);
-  key_add(k, g_scr.ux);
-  key_add(k, g_scr.uy);
-  key_add(k, g_scr.ux2);
-  key_add(k, g_scr.uy2);
-  key_add(k, g_scr.p);
+  key_add(k, scr.vof);
+  key_add(k, scr.ux);
+  key_add(k, scr.uy);
+  key_add(k, scr.ux2);
+  key_add(k, scr.uy2);
+  key_add(k, scr.p);
   k.v.push_back(march_fold() ? 1 : 0);
   key_add(k, cf.rhf);
   key_add(k, rhs);
@@ -768,28 +832,17 @@ static StepKey step_key(const DomainCtx* c, fluid_t* f, interface_t* s, const Co
   k.v.push_back((uint64_t)options().gauge | ((uint64_t)options().tdm << 8) |
                 ((uint64_t)options().chunk << 16) | ((uint64_t)options().precision << 48) |
                 ((uint64_t)options().curvature << 56));
-  key_add(k, g_scr.kappa);
-  for (const unsigned* l : g_scr.klist) key_add(k, l);
-  k.v.push_back((uint64_t)(int64_t)g_scr.klast);
-  key_add(k, g_scr.cut);
+  key_add(k, scr.kappa);
+  for (const unsigned* l : scr.klist) key_add(k, l);
+  k.v.push_back((uint64_t)(int64_t)scr.klast);
+  key_add(k, scr.cut);
   k.v.push_back(march_ordered(options().precision == SBFS_PRECISION_MIXED) ? 1 : 0);
   k.v.push_back(stream_fields(c->nx, c->ny) ? 1 : 0);
-  key_add(k, g_scr.order);
-  k.v.push_back(graph_epoch());
+  key_add(k, scr.order);
+  k.v.push_back(c->epoch);
+  k.v.push_back(poisson_epoch(c));
   return k;
 }
-
-struct StepGraph {
-  StepKey key;
-  hipGraphExec_t exec = nullptr;
-  // state pointers after the step, then the scratch vof and pressure, which
-  // a step swaps with the state's (the pressure once per step)
-  void* after[kStateArrays + 2] = {};
-  uint64_t last_use = 0;
-};
-static StepGraph g_graph[2];
-static StepKey g_seen[2];
-static uint64_t g_clock = 0;
 
 static bool graphs_enabled() {
   static int on = -1;
@@ -803,25 +856,31 @@ static bool graphs_enabled() {
 static int step_graph(const domain_t* domain, DomainCtx* c, fluid_t* fluid, interface_t* interface,
                       const Coef& cf, double* rhs, int band, double learned_h) {
   if (!graphs_enabled()) return fused_body(domain, c, fluid, interface, cf, rhs, band, learned_h);
+  FusedState& fs = *c->fused;
+  FusedScratch& scr = fs.scr;
   const StepKey key = step_key(c, fluid, interface, cf, rhs, band);
-  g_clock++;
-  for (StepGraph& g : g_graph) {
+  fs.clock++;
+  for (StepGraph& g : fs.graph) {
     if (g.exec && g.key == key) {
       SBFS_HIP(hipGraphLaunch(g.exec, stream()));
       for (int n = 0; n < kStateArrays; n++) state_arrays(fluid, interface, n)->data = g.after[n];
-      g_scr.vof = (double*)g.after[kStateArrays];
-      g_scr.p = (double*)g.after[kStateArrays + 1];
-      g.last_use = g_clock;
+      scr.vof = (double*)g.after[kStateArrays];
+      scr.p = (double*)g.after[kStateArrays + 1];
+      g.last_use = fs.clock;
       return 0;
     }
   }
-  const bool seen = g_seen[0] == key || g_seen[1] == key;
+  bool seen = false;
+  for (const StepKey& k : fs.seen) seen = seen || k == key;
   if (!seen) {
     // first sight of this configuration: run eagerly (builds plans / tables)
-    g_seen[g_clock & 1] = key;
+    fs.seen[fs.clock % kStepGraphs] = key;
     return fused_body(domain, c, fluid, interface, cf, rhs, band, learned_h);
   }
-  StepGraph& g = g_graph[0].last_use <= g_graph[1].last_use ? g_graph[0] : g_graph[1];
+  StepGraph* slot = &fs.graph[0];
+  for (StepGraph& g : fs.graph)
+    if (g.last_use < slot->last_use) slot = &g;
+  StepGraph& g = *slot;
   if (g.exec) {
     (void)hipGraphExecDestroy(g.exec);
     g.exec = nullptr;
@@ -840,9 +899,9 @@ static int step_graph(const domain_t* domain, DomainCtx* c, fluid_t* fluid, inte
   SBFS_HIP(ie);
   g.key = key;
   for (int n = 0; n < kStateArrays; n++) g.after[n] = state_arrays(fluid, interface, n)->data;
-  g.after[kStateArrays] = g_scr.vof;
-  g.after[kStateArrays + 1] = g_scr.p;
-  g.last_use = g_clock;
+  g.after[kStateArrays] = scr.vof;
+  g.after[kStateArrays + 1] = scr.p;
+  g.last_use = fs.clock;
   SBFS_HIP(hipGraphLaunch(g.exec, stream()));
   return 0;
 }
@@ -862,7 +921,8 @@ int integrate_fused(const domain_t* domain, fluid_t* fluid, interface_t* interfa
   if (check_array(domain, &interface->vof, NA_VOF, 8, "vof")) return 1;
   for (int n = 0; n < 2; n++)
     if (check_array(domain, &interface->src[n], NA_SRC, 8, "src")) return 1;
-  if (scratch(domain, interface, fluid)) return 1;
+  if (!c->fused) c->fused = new FusedState();
+  if (scratch(c, interface, fluid, options().curvature == SBFS_CURVATURE_LEARNED)) return 1;
   Coef cf;
   if (coef_tables(domain, c, fluid->Re, &cf)) return 1;
   const int nx = (int)c->nx, ny = (int)c->ny;
@@ -871,7 +931,7 @@ int integrate_fused(const domain_t* domain, fluid_t* fluid, interface_t* interfa
   const int band = march_band(nx, ny, options().precision == SBFS_PRECISION_MIXED);
   if (band <= 0) return 1;
   if (march_ordered(options().precision == SBFS_PRECISION_MIXED) &&
-      order_buffers(march_units(nx, ny, band)))
+      order_buffers(c, march_units(nx, ny, band)))
     return 1;
   if (load_dt_coefs()) return 1;
   double learned_h = 0.;

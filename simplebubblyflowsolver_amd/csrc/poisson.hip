@@ -37,7 +37,6 @@ static const double kPiPoisson = 3.14159265358979324;  // compute_potential.c:21
 
 void poisson_destroy(PoissonPlan* p) {
   if (!p) return;
-  graph_epoch_bump();
   (void)hipFree(p->buf);
   (void)hipFree(p->v);
   (void)hipFree(p->q1);
@@ -929,6 +928,7 @@ static PoissonPlan* plan_get(const domain_t* d, DomainCtx* c) {
   if (c->poisson) {
     poisson_destroy(c->poisson);
     c->poisson = nullptr;
+    c->epoch++;
   }
   if (nx < 2 || (nx & (nx - 1)) != 0 || nx > 4096) {
     set_error("Poisson solver: Nx = %d must be a power of two in [2, 4096]", nx);
@@ -950,6 +950,8 @@ static PoissonPlan* plan_get(const domain_t* d, DomainCtx* c) {
   c->poisson = p;
   return p;
 }
+
+uint64_t poisson_epoch(const DomainCtx* c) { return c->poisson ? c->poisson->epoch : 0; }
 
 static int row_threads(int m) { return m >= 1024 ? 512 : 256; }
 

@@ -29,6 +29,7 @@ struct PoissonPlan {
   double2* t2 = nullptr;     // n      e^{-i pi k/(2n)}
   // partitioned solver
   int L = 0, P = 0;
+  uint64_t epoch = 0;        // moves when the tables below are replaced
   double a = 0.;             // off-diagonal 1/hy^2
   double* ptab = nullptr;    // [4][K][nx]: inv, v, w, z per (row-in-chunk, mode)
   double* htab = nullptr;    // [P][nx]: first column of the reduced circulant's inverse

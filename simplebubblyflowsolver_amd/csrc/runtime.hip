@@ -164,15 +164,12 @@ static uint64_t domain_hash(const domain_t* d) {
 }
 
 void poisson_destroy(PoissonPlan* p);  // poisson.hip
-
-static uint64_t g_graph_epoch = 0;
-void graph_epoch_bump() { g_graph_epoch++; }
-uint64_t graph_epoch() { return g_graph_epoch; }
+void fused_destroy(FusedState* s);     // fused.hip
 
 static void ctx_free(DomainCtx* c) {
   if (!c) return;
   (void)hipStreamSynchronize(g_stream);
-  graph_epoch_bump();
+  fused_destroy(c->fused);
   (void)hipFree(c->hxxf);
   (void)hipFree(c->hxxc);
   (void)hipFree(c->jdxf);

@@ -104,6 +104,7 @@ constexpr double kUyXp = 0.;        // src/param/boundary-condition.c:4
 // device state per domain
 // ---------------------------------------------------------------------------
 struct PoissonPlan;  // poisson.hip
+struct FusedState;   // fused.hip
 
 struct DomainCtx {
   // identity of the host domain this mirrors
@@ -121,7 +122,15 @@ struct DomainCtx {
   double* dt_dev = nullptr;  // device-resident dt (1 double)
   double* host_pin = nullptr;  // pinned host staging (16 doubles)
   PoissonPlan* poisson = nullptr;
+  FusedState* fused = nullptr;
+  // The domain's captured step graphs hold device addresses that their keys do
+  // not list (the Poisson plan's buffers, the stage arguments).  Whatever frees
+  // or reuses such memory moves this epoch (PoissonPlan::epoch for the plan's
+  // tables), which is part of every key, so no graph replays against memory that
+  // was freed, even when a new allocation has the old addresses.
+  uint64_t epoch = 0;
 };
+uint64_t poisson_epoch(const DomainCtx* c);  // poisson.hip
 
 constexpr int kRedBlocks = 1024;          // partial-reduction blocks
 constexpr int kRedSlots = kRedBlocks * 8 + 64;
@@ -189,14 +198,6 @@ int curv_field_init(float* kappa, unsigned* const* lists, int nlists, long cells
 // with this vof (march.hpp), which the gate then reads instead of the vof.
 int curv_mlp_launch(const double* vof, const unsigned long long* cut, float* kappa, unsigned* list,
                     const unsigned* prev, unsigned* next, int nx, int ny, double h, hipStream_t st);
-// Captured step graphs hold device addresses that their keys do not list
-// (Poisson plan buffers, domain metrics).
-// Whatever frees such memory bumps this epoch, which is part of every key,
-// so no graph replays against freed memory, even when a new allocation
-// reuses the old addresses.
-void graph_epoch_bump();
-uint64_t graph_epoch();
-
 // kernel timing (profiler.hip): events around launches while profiling
 bool prof_active();  // kernel timing on (sbfs_profile_start)
 void prof_begin(const char* name);
