@@ -84,6 +84,7 @@ struct sbfs_ensemble {
   unsigned nb_dt = 0, nb_march = 0, nb_row = 0, nb_mode = 0, nb_post = 0, nb_part = 0, nb_conv = 0, nb_col = 0;
   unsigned off_march = 0, off_row = 0, off_mode = 0, off_post = 0, off_part = 0, off_conv = 0, off_col = 0;
   size_t lds = 0, lds_conv = 0, lds_col = 0;
+  int tile = 0;  // tile height of the stage kernel (0: the marching one, bands of `band`)
   int row_threads = 64;
   double* dts = nullptr;
   hipGraphExec_t graph[2] = {};
@@ -144,10 +145,17 @@ static int plan(sbfs_ensemble* e) {
   };
   for (int c = 0; c < n; c++) add(c, (unsigned)steps[0][c].dt.nblk);
   e->nb_dt = (unsigned)map.size();
+  unsigned groups[2] = {0, 0};
+  for (auto& k : e->cs) {
+    groups[0] += tile_groups((int)k.ctx->nx, (int)k.ctx->ny, kTileShort);
+    groups[1] += tile_groups((int)k.ctx->nx, (int)k.ctx->ny, kTileTall);
+  }
+  // (the results do not depend on it, so a later change of the precision keeps it)
+  e->tile = tile_rows(groups[0], groups[1], options().precision == SBFS_PRECISION_MIXED);
   e->off_march = (unsigned)map.size();
   for (int c = 0; c < n; c++) {
     const auto& m = steps[0][c].march[0];
-    add(c, cdiv(m.nx, kStrip) * cdiv(m.ny, m.band));
+    add(c, e->tile ? tile_groups(m.nx, m.ny, e->tile) : cdiv(m.nx, kStrip) * cdiv(m.ny, m.band));
   }
   e->nb_march = (unsigned)map.size() - e->off_march;
   e->off_row = (unsigned)map.size();
@@ -246,7 +254,9 @@ static int launch_step(sbfs_ensemble* e, int p) {
     const MarchArgs* ma = e->march[p] + (size_t)k * n;
     const RowArgs* ro = e->rows[p] + (size_t)k * n;
     const uint2* mm = mp + e->off_march;
-    if (mixed && k > 0)
+    if (e->tile)
+      tile_launch_batch(ma, mm, e->nb_march, e->tile, mixed, k > 0);
+    else if (mixed && k > 0)
       SBFS_TIMED("k_march_mixed_corr",
                  hipLaunchKernelGGL(k_march_mixed_corr_batch, dim3(e->nb_march), dim3(64), 0, stream(), ma, mm));
     else if (mixed)

@@ -465,6 +465,27 @@ static bool march_ordered(bool mixed) {
   return !mixed;
 }
 
+// The tile height of the small grids' stage kernel (tile.hip), 0 for the
+// marching kernel.  The short tile while its workgroups all run at once (two per
+// CU, 512: 256 x 256 has 430, 256 x 512 would take 855 and is faster with 235
+// tall ones, 63 against 74 us per step).  The tall one for up to four rounds of
+// one per CU in FP64 and two and a half in mixed precision, where the marching
+// kernel's lower redundancy catches up (512 x 1024, 846 tall tiles: 153 against
+// 173 us in FP64, 129 against 128 mixed; 1024 x 1024, 1692: 260 against 241 and
+// 218 against 179).  SBFS_MARCH_TILE=0 takes the marching kernel, =3 or =11 the
+// tile of that height (the results are bitwise the same).
+int tile_rows(unsigned short_groups, unsigned tall_groups, bool mixed) {
+  if (const char* e = getenv("SBFS_MARCH_TILE")) {
+    const int h = atoi(e);
+    return h == kTileShort || h == kTileTall ? h : 0;
+  }
+  if (short_groups <= 512) return kTileShort;
+  return tall_groups <= (mixed ? 640u : 1024u) ? kTileTall : 0;
+}
+static int tile_rows(int nx, int ny, bool mixed) {
+  return tile_rows(tile_groups(nx, ny, kTileShort), tile_groups(nx, ny, kTileTall), mixed);
+}
+
 // Rows per band of k_march.  Every wavefront marches its band plus kWarm + 2
 // rows of ring fill, and a wavefront lives for the whole band, so the grid
 // is sized in rounds of the device: multiples of the resident wavefront
@@ -696,7 +717,8 @@ static int fused_body(const domain_t* domain, DomainCtx* c, fluid_t* fluid, inte
   // them (the previous step's; the bubbles move a fraction of a cell per
   // step), for all three stages of this step
   const bool mixed = options().precision == SBFS_PRECISION_MIXED;
-  const bool ordered = march_ordered(mixed);
+  const int tile = tile_rows(nx, ny, mixed);
+  const bool ordered = tile == 0 && march_ordered(mixed);
   const int units = march_units(nx, ny, band);
   if (ordered) {
     SBFS_REQUIRE(scr.units >= units, "integrate: no dispatch-order buffers for %d units", units);
@@ -737,7 +759,9 @@ static int fused_body(const domain_t* domain, DomainCtx* c, fluid_t* fluid, inte
       const dim3 grid = ordered ? dim3(units) : dim3(cdiv(nx, kStrip), cdiv(ny, band)), block(64);
       const MarchArgs* ma = nullptr;
       if (device_args(c, m, &ma)) return 1;
-      if (mixed && corr)
+      if (tile) {
+        tile_launch(ma, nx, ny, tile, mixed, corr);
+      } else if (mixed && corr)
         SBFS_TIMED("k_march_mixed_corr", hipLaunchKernelGGL(k_march_mixed_corr, grid, block, 0, stream(), ma));
       else if (mixed)
         SBFS_TIMED("k_march_mixed", hipLaunchKernelGGL(k_march_mixed, grid, block, 0, stream(), ma));
@@ -836,7 +860,8 @@ static StepKey step_key(const DomainCtx* c, fluid_t* f, interface_t* s, const Co
   for (const unsigned* l : scr.klist) key_add(k, l);
   k.v.push_back((uint64_t)(int64_t)scr.klast);
   key_add(k, scr.cut);
-  k.v.push_back(march_ordered(options().precision == SBFS_PRECISION_MIXED) ? 1 : 0);
+  const bool mixed = options().precision == SBFS_PRECISION_MIXED;
+  k.v.push_back((march_ordered(mixed) ? 1 : 0) | ((uint64_t)tile_rows((int)c->nx, (int)c->ny, mixed) << 1));
   k.v.push_back(stream_fields(c->nx, c->ny) ? 1 : 0);
   key_add(k, scr.order);
   k.v.push_back(c->epoch);
@@ -930,7 +955,8 @@ int integrate_fused(const domain_t* domain, fluid_t* fluid, interface_t* interfa
   if (poisson_transform_fused(domain, c, fluid, &rhs)) return 1;
   const int band = march_band(nx, ny, options().precision == SBFS_PRECISION_MIXED);
   if (band <= 0) return 1;
-  if (march_ordered(options().precision == SBFS_PRECISION_MIXED) &&
+  const bool mixed = options().precision == SBFS_PRECISION_MIXED;
+  if (march_ordered(mixed) && tile_rows(nx, ny, mixed) == 0 &&
       order_buffers(c, march_units(nx, ny, band)))
     return 1;
   if (load_dt_coefs()) return 1;

@@ -22,6 +22,12 @@ constexpr int kStrip = 58;
 // match with the staged one.)
 constexpr int kWarm = 4;
 constexpr int kWarmCorr = 4;
+// Output rows of a workgroup of the small grids' stage kernel (tile.hip): the
+// short tile has the shorter latency, the tall one less redundant work.
+constexpr int kTileShort = 3, kTileTall = 11;
+inline unsigned tile_groups(int nx, int ny, int rows) {
+  return cdiv(nx, kStrip) * cdiv(ny, rows);
+}
 
 // per-column quotients of the metrics (see fused.hip)
 struct Coef {
@@ -158,6 +164,11 @@ __global__ void k_march_batch(const MarchArgs* tab, const uint2* map);
 __global__ void k_march_corr_batch(const MarchArgs* tab, const uint2* map);
 __global__ void k_march_mixed_batch(const MarchArgs* tab, const uint2* map);
 __global__ void k_march_mixed_corr_batch(const MarchArgs* tab, const uint2* map);
+// tile.hip; tile_rows (fused.hip): the tile's height for so many workgroups of
+// short and tall tiles, 0 for the marching kernel
+int tile_rows(unsigned short_groups, unsigned tall_groups, bool mixed);
+void tile_launch(const MarchArgs* ma, int nx, int ny, int rows, bool mixed, bool corr);
+void tile_launch_batch(const MarchArgs* tab, const uint2* map, unsigned blocks, int rows, bool mixed, bool corr);
 __global__ void k_post_batch(const PostArgs* tab, const uint2* map);
 
 }  // namespace sbfs
