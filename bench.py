@@ -67,7 +67,7 @@ BYTES_PER_CELL = {
     "k_stress": 56, "k_rhs_ux": 80, "k_rhs_uy": 72, "k_predict_ux": 56, "k_predict_uy": 56,
     "k_dct2_rhs": 40, "k_tdm_sequential": 16, "k_part_reduce": 16, "k_part_conv": 0,
     "k_dct3_psi": 16, "k_correct_ux": 40, "k_correct_uy": 40,
-    "k_update_p": 24, "k_dt_partial": 16, "k_dt_final": 0,
+    "k_update_p": 24, "k_dt": 16,
     # fused path
     # (stages 1 and 2: 9 reads + 7 writes each; the mixed kernels keep the
     # momentum sources as FP32: 8 bytes fewer per cell in stage 0, and 16 and

@@ -51,11 +51,6 @@ static void set_state(fluid_t* f, interface_t* s, CaseScratch* scr, const CaseSt
   *scr = st.scr;
 }
 
-__global__ void k_gather_dt(const DtArgs* __restrict__ tab, int n, double* __restrict__ out) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c < n) out[c] = *tab[c].dt;
-}
-
 }  // namespace sbfs
 
 using namespace sbfs;
@@ -86,7 +81,7 @@ struct sbfs_ensemble {
   size_t lds = 0, lds_conv = 0, lds_col = 0;
   int tile = 0;  // tile height of the stage kernel (0: the marching one, bands of `band`)
   int row_threads = 64;
-  double* dts = nullptr;
+  double* dts = nullptr;  // pinned: every case's dt, written by k_dt_batch
   hipGraphExec_t graph[2] = {};
   int runs[2] = {};
   int graph_precision = -1;
@@ -134,7 +129,7 @@ static int plan(sbfs_ensemble* e) {
     k.start[0] = st;
     for (int p = 0; p < 2; p++) {
       if (p == 1) k.start[1] = st;
-      if (ensemble_plan_step(&k.d, k.ctx, &st.f, &st.s, k.cf, e->band, st.scr, steps[p][c])) return 1;
+      if (ensemble_plan_step(&k.d, k.ctx, &st.f, &st.s, k.cf, e->band, e->dts + c, st.scr, steps[p][c])) return 1;
     }
     SBFS_REQUIRE(same_state(st, k.start[0]), "ensemble: the step's pointer state does not return after two steps");
   }
@@ -246,10 +241,8 @@ static int launch_step(sbfs_ensemble* e, int p) {
   const int n = (int)e->cs.size();
   const bool mixed = options().precision == SBFS_PRECISION_MIXED;
   const uint2* mp = e->maps;
-  SBFS_TIMED("k_dt_partial", hipLaunchKernelGGL(k_dt_partial_batch, dim3(e->nb_dt), dim3(kRedThreads), 0, stream(),
-                                                (const DtArgs*)e->dt[p], mp));
-  SBFS_TIMED("k_dt_final",
-             hipLaunchKernelGGL(k_dt_final_batch, dim3(n), dim3(kRedThreads), 0, stream(), (const DtArgs*)e->dt[p]));
+  SBFS_TIMED("k_dt", hipLaunchKernelGGL(k_dt_batch, dim3(e->nb_dt), dim3(kRedThreads), 0, stream(),
+                                        (const DtArgs*)e->dt[p], mp));
   for (int k = 0; k < 3; k++) {
     const MarchArgs* ma = e->march[p] + (size_t)k * n;
     const RowArgs* ro = e->rows[p] + (size_t)k * n;
@@ -391,7 +384,11 @@ extern "C" int sbfs_ensemble_create(const sbfs_case_t* cases, int n, sbfs_ensemb
     sbfs_ensemble_destroy(e);
     return 1;
   }
-  SBFS_HIP(hipMalloc(&e->dts, sizeof(double) * n));
+  if (hipHostMalloc(&e->dts, sizeof(double) * n, 0) != hipSuccess) {
+    set_error("sbfs_ensemble_create: out of pinned memory");
+    sbfs_ensemble_destroy(e);
+    return 1;
+  }
   *out = e;
   return 0;
 }
@@ -410,14 +407,8 @@ extern "C" int sbfs_ensemble_step(sbfs_ensemble_t* e, double* dts) {
   if (!e->planned && plan(e)) return 1;
   if (run_step(e)) return 1;
   const int n = (int)e->cs.size();
-  if (dts) {
-    // the dt of the step just taken (the tables of its parity)
-    hipLaunchKernelGGL(k_gather_dt, dim3(cdiv(n, 64)), dim3(64), 0, stream(), (const DtArgs*)e->dt[e->parity ^ 1], n,
-                       e->dts);
-    if (check_launch("sbfs_ensemble_step: dt")) return 1;
-    SBFS_HIP(hipMemcpyAsync(dts, e->dts, sizeof(double) * n, hipMemcpyDeviceToHost, stream()));
-  }
   SBFS_HIP(hipStreamSynchronize(stream()));
+  if (dts) memcpy(dts, e->dts, sizeof(double) * n);
   return 0;
 }
 
@@ -494,7 +485,7 @@ extern "C" int sbfs_ensemble_destroy(sbfs_ensemble_t* e) {
     if (k.f.ux.data) sbfs_fluid_destroy(&k.f);
     if (k.d.xf) sbfs_domain_destroy(&k.d);
   }
-  (void)hipFree(e->dts);
+  (void)hipHostFree(e->dts);
   delete e;
   return 0;
 }

@@ -710,7 +710,7 @@ static int fused_body(const domain_t* domain, DomainCtx* c, fluid_t* fluid, inte
   };
   if (overlap && fork_curv(0, D(interface->vof))) return 1;
   if (compute_dt_device(domain, c, fluid, interface)) return 1;
-  const double* dtp = c->dt_dev;
+  const double* dtp = &c->dt->dt;
   const bool fold = march_fold();
   const bool nt = stream_fields(nx, ny);  // streaming accesses of the rows touched once
   // the units in order of the interface rows the last stage kernel found in
@@ -971,9 +971,8 @@ int integrate_fused(const domain_t* domain, fluid_t* fluid, interface_t* interfa
     learned_h = h;
   }
   if (step_graph(domain, c, fluid, interface, cf, rhs, band, learned_h)) return 1;
-  SBFS_HIP(hipMemcpyAsync(c->host_pin, c->dt_dev, sizeof(double), hipMemcpyDeviceToHost, stream()));
   SBFS_HIP(hipStreamSynchronize(stream()));
-  *dt = c->host_pin[0];
+  *dt = *dt_host(c);
   return 0;
 }
 
@@ -983,9 +982,9 @@ int integrate_fused(const domain_t* domain, fluid_t* fluid, interface_t* interfa
 // recording the arguments of every launch.  On return the structs and
 // scratch hold the pointer state after the step.
 int ensemble_plan_step(const domain_t* domain, DomainCtx* c, fluid_t* fluid, interface_t* interface,
-                       const Coef& cf, int band, CaseScratch& scr, CaseStep& out) {
-  if (dt_args(domain, c, fluid, interface, &out.dt)) return 1;
-  const double* dtp = c->dt_dev;
+                       const Coef& cf, int band, double* host_dt, CaseScratch& scr, CaseStep& out) {
+  if (dt_args(domain, c, fluid, interface, c->dt, host_dt, &out.dt)) return 1;
+  const double* dtp = &c->dt->dt;
   double* rhs = nullptr;
   if (poisson_transform_fused(domain, c, fluid, &rhs)) return 1;
   double* const us[3] = {scr.ux[0], scr.ux[1], scr.ux[0]};

@@ -159,7 +159,7 @@ struct CaseStep {
 };
 int coef_build(const domain_t* d, double Re, double** buf, Coef* out);
 int ensemble_plan_step(const domain_t* domain, DomainCtx* c, fluid_t* fluid, interface_t* interface,
-                       const Coef& cf, int band, CaseScratch& scr, CaseStep& out);
+                       const Coef& cf, int band, double* host_dt, CaseScratch& scr, CaseStep& out);
 __global__ void k_march_batch(const MarchArgs* tab, const uint2* map);
 __global__ void k_march_corr_batch(const MarchArgs* tab, const uint2* map);
 __global__ void k_march_mixed_batch(const MarchArgs* tab, const uint2* map);

@@ -176,7 +176,7 @@ static void ctx_free(DomainCtx* c) {
   (void)hipFree(c->jdxc);
   (void)hipFree(c->xc);
   (void)hipFree(c->red);
-  (void)hipFree(c->dt_dev);
+  (void)hipFree(c->dt);
   (void)hipHostFree(c->host_pin);
   poisson_destroy(c->poisson);
   delete c;
@@ -234,7 +234,8 @@ DomainCtx* domain_ctx(const domain_t* d) {
             hipMalloc(&c->jdxc, sizeof(double) * nx) == hipSuccess &&
             hipMalloc(&c->xc, sizeof(double) * (nx + 2)) == hipSuccess &&
             hipMalloc(&c->red, sizeof(double) * kRedSlots) == hipSuccess &&
-            hipMalloc(&c->dt_dev, sizeof(double) * 8) == hipSuccess &&
+            hipMalloc(&c->dt, sizeof(DtSlot)) == hipSuccess &&
+            hipMemset(c->dt, 0, sizeof(DtSlot)) == hipSuccess &&
             hipHostMalloc(&c->host_pin, sizeof(double) * 16, 0) == hipSuccess;
   if (!ok || upload_metrics(d, c)) {
     set_error("device allocation for the domain failed");

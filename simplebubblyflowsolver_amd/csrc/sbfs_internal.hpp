@@ -106,6 +106,18 @@ constexpr double kUyXp = 0.;        // src/param/boundary-condition.c:4
 struct PoissonPlan;  // poisson.hip
 struct FusedState;   // fused.hip
 
+// decide_dt's result on the device and the words its workgroups combine their
+// minima in (step.hip), which are 0 between launches
+constexpr unsigned kDtWords = 32, kDtFlat = 128;
+struct alignas(128) DtWord {
+  unsigned long long key;
+  unsigned count;
+};
+struct DtSlot {
+  double dt;
+  DtWord word[1 + kDtWords];
+};
+
 struct DomainCtx {
   // identity of the host domain this mirrors
   size_t nx = 0, ny = 0;
@@ -119,8 +131,8 @@ struct DomainCtx {
   double* xc = nullptr;    // nx+2
   // scratch for reductions
   double* red = nullptr;   // kRedSlots doubles
-  double* dt_dev = nullptr;  // device-resident dt (1 double)
-  double* host_pin = nullptr;  // pinned host staging (16 doubles)
+  DtSlot* dt = nullptr;    // device-resident dt
+  double* host_pin = nullptr;  // pinned host staging (16 doubles, the last the step's dt)
   PoissonPlan* poisson = nullptr;
   FusedState* fused = nullptr;
   // The domain's captured step graphs hold device addresses that their keys do
@@ -131,6 +143,8 @@ struct DomainCtx {
   uint64_t epoch = 0;
 };
 uint64_t poisson_epoch(const DomainCtx* c);  // poisson.hip
+
+inline double* dt_host(const DomainCtx* c) { return c->host_pin + 15; }
 
 constexpr int kRedBlocks = 1024;          // partial-reduction blocks
 constexpr int kRedSlots = kRedBlocks * 8 + 64;
@@ -209,20 +223,20 @@ void prof_end();
     ::sbfs::prof_end();       \
   } while (0)
 
-// arguments of one case's decide_dt kernels in an ensemble (step.hip)
+// arguments of decide_dt's kernel (step.hip)
 struct DtArgs {
   const double* ux;
   const double* uy;
   const double* hxxf;
   double hy, cadv, dif0, dif1, dint;
-  double* partial;
-  double* dt;
+  DtSlot* slot;
+  double* host;
   int nx, ny, rows, gx, nblk;
-  int stream;  // streaming loads (stream_fields)
 };
-int dt_args(const domain_t* d, DomainCtx* c, const fluid_t* f, const interface_t* s, DtArgs* a);
-__global__ void k_dt_partial_batch(const DtArgs* tab, const uint2* map);
-__global__ void k_dt_final_batch(const DtArgs* tab);
+int dt_args(const domain_t* d, const DomainCtx* c, const fluid_t* f, const interface_t* s, DtSlot* slot, double* host,
+            DtArgs* a);
+int dt_launch(const DtArgs& a);
+__global__ void k_dt_batch(const DtArgs* tab, const uint2* map);
 
 // grid-dimension helpers
 inline unsigned cdiv(long a, long b) { return (unsigned)((a + b - 1) / b); }
@@ -236,9 +250,6 @@ int poisson_solve(const domain_t* d, DomainCtx* c, double dt_old,
                   double dt_new, fluid_t* f);
 int compute_dt_device(const domain_t* d, DomainCtx* c, const fluid_t* f,
                       const interface_t* s);
-int dt_grid(int nx, int ny, int capacity, int* rows, int* nblk);
-int dt_launch(const domain_t* d, const DomainCtx* c, const fluid_t* f, const interface_t* s,
-              int capacity, double* partial, double* dt_out);
 // the domain's device context if one exists and is current, without
 // creating or refreshing one (nullptr otherwise)
 DomainCtx* domain_ctx_find(const domain_t* d);

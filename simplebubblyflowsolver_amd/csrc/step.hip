@@ -1,5 +1,6 @@
 // Time-step control (reference src/decide_dt.c), device diagnostics and the
 // integrator (src/integrate.c).
+#include <algorithm>
 #include <cfloat>
 #include <cmath>
 
@@ -17,128 +18,102 @@ static const double kPiDt = 3.1415926535897932384626433832;  // decide_dt.c:16
 static const double kDtMax = 1.;                              // decide_dt.c:25
 
 
-// advective limit min over faces of h / (|u| + small) (decide_dt.c:49-64)
-// advective limit min over faces of h / (|u| + small) (decide_dt.c:49-64):
-// a workgroup takes kRedThreads consecutive columns of `rows` rows (16, or
-// more when the partial minima would not fit the reduction buffer), each
-// thread one column, so the loads of a thread are independent and in flight
-// together; a min does not depend on the combination order
+// decide_dt in one launch: the advective limit, min over faces of
+// h / (|u| + small) (decide_dt.c:49-64), and its combination with the other
+// limits (:157-167).  A workgroup takes kRedThreads consecutive columns of `rows`
+// rows, each thread one column, so the loads of a thread are independent and in
+// flight together; its minimum m joins the others through an atomic, and the
+// last workgroup writes dt to device memory, for the step's kernels, and to
+// pinned host memory, for the caller.  (As a second launch and a copy queued after
+// the step, the combination and the caller's dt cost 10 us of a 138 us step at
+// 64 x 128.)  A min does not depend on the combination order.
+// DtWord::key holds the largest ~bits(m): m is positive and no NaN, so its bits
+// grow with it, and 0 is the identity.  A workgroup adds to the counter after
+// its update of the key has returned, that is, has been performed where every XCD
+// sees it, so the workgroup that counts the last sees every minimum, and returns
+// both words to 0 for the next launch.  Updates of one address take about 10 ns
+// each, one after another (k_dt of 2048 workgroups on one pair of words: 74 us at
+// 2048 x 4096), so above kDtFlat workgroups they combine in kDtWords groups first,
+// each on its own cache lines, and the last of each group in the first pair.
+// (Stored partial minima with an acquire / release counter, whose cache
+// write-backs and invalidations every workgroup pays, took 76 us there.)
+template <int B, bool NT>
+__device__ __forceinline__ double dt_column(const DtArgs& a, int i, int j0) {
+  // The column's minimum of h / (|u| + small) is h over its largest
+  // |u| + small, bit for bit: a correctly rounded quotient does not grow
+  // with its divisor, so the largest divisor gives the smallest quotient
+  // (and fmax passes over a NaN as fmin does).  One division per field
+  // and thread instead of one per cell.
+  const double small = 1.e-8;
+  double mx = 0., my = 0.;
+  // rows past ny repeat row ny (a repeated value leaves a max unchanged),
+  // so the loads carry no branch and are all in flight together; with NT
+  // they are streaming loads (read once; 124 -> 88 us at 4096 x 8192, see
+  // stream_fields)
+  auto ld = [](const double* p) {
+    if constexpr (NT) return __builtin_nontemporal_load(p);
+    else return *p;
+  };
+  for (int r0 = 0; r0 < a.rows; r0 += B) {
+#pragma unroll
+    for (int r = 0; r < B; r++) {
+      const int j = min(j0 + r0 + r, a.ny);
+      if (i >= 2) mx = fmax(mx, fabs(ld(a.ux + L::xf(i, j, a.nx))) + small);
+      my = fmax(my, fabs(ld(a.uy + L::cc(i, j, a.nx))) + small);
+    }
+  }
+  double m = kDtMax;
+  if (i >= 2) m = fmin(m, a.hxxf[i - 1] / mx);
+  return fmin(m, a.hy / my);
+}
 
 template <bool NT>
-__device__ __forceinline__ void dt_partial_body(const double* __restrict__ ux, const double* __restrict__ uy,
-                                                const double* __restrict__ hxxf, double hy, int nx, int ny,
-                                                int rows, double* __restrict__ partial, int bx, int by, int gx) {
+__device__ __forceinline__ void dt_body(const DtArgs& a, int bx, int by) {
   __shared__ double sh[kRedThreads / 64];
-  const double small = 1.e-8;
   double m = kDtMax;
   const int i = 1 + (int)(bx * kRedThreads + threadIdx.x);
-  const int j0 = 1 + by * rows;
-  if (i <= nx) {
-    const double hx = hxxf[i - 1];
-    // The column's minimum of h / (|u| + small) is h over its largest
-    // |u| + small, bit for bit: a correctly rounded quotient does not grow
-    // with its divisor, so the largest divisor gives the smallest quotient
-    // (and fmax passes over a NaN as fmin does).  One division per field
-    // and thread instead of one per cell.
-    double mx = 0., my = 0.;
-    // rows past ny repeat row ny (a repeated value leaves a max unchanged),
-    // so the loads carry no branch and are all in flight together; with NT
-    // they are streaming loads (read once; 124 -> 88 us at 4096 x 8192, see
-    // stream_fields)
-    auto ld = [](const double* p) {
-      if constexpr (NT) return __builtin_nontemporal_load(p);
-      else return *p;
-    };
-#pragma unroll 16
-    for (int r = 0; r < rows; r++) {
-      const int j = min(j0 + r, ny);
-      if (i >= 2) mx = fmax(mx, fabs(ld(ux + L::xf(i, j, nx))) + small);
-      my = fmax(my, fabs(ld(uy + L::cc(i, j, nx))) + small);
-    }
-    if (i >= 2) m = fmin(m, hx / mx);
-    m = fmin(m, hy / my);
-  }
+  const int j0 = 1 + by * a.rows;
+  if (i <= a.nx) m = a.rows >= 16 ? dt_column<16, NT>(a, i, j0) : dt_column<4, NT>(a, i, j0);
   m = block_reduce<0>(m, sh);
-  if (threadIdx.x == 0) partial[by * gx + bx] = m;
+  if (threadIdx.x != 0) return;
+  unsigned long long key = ~(unsigned long long)__double_as_longlong(m);
+  // joins the key of `n` workgroups; true for the last, with the joined key
+  auto join = [&key](DtWord* w, unsigned n) {
+    unsigned long long old = __hip_atomic_fetch_max(&w->key, key, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    // (an empty statement that reads the update's return: the wait for it comes
+    // here, before the counter's update, which stays behind the statement)
+    asm volatile("" : "+v"(old)::"memory");
+    if (__hip_atomic_fetch_add(&w->count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u != n) return false;
+    key = __hip_atomic_exchange(&w->key, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(&w->count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return true;
+  };
+  unsigned groups = (unsigned)a.nblk;
+  if (groups > kDtFlat) {
+    const unsigned g = (unsigned)(by * a.gx + bx) % kDtWords;
+    if (!join(&a.slot->word[1 + g], (groups - g + kDtWords - 1) / kDtWords)) return;
+    groups = kDtWords;
+  }
+  if (!join(&a.slot->word[0], groups)) return;
+  double r = __longlong_as_double((long long)~key) * a.cadv;
+  r = fmin(r, a.dif0);
+  r = fmin(r, a.dif1);
+  r = fmin(r, a.dint);
+  a.slot->dt = r;
+  __hip_atomic_store(a.host, r, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 template <bool NT>
-__global__ __launch_bounds__(kRedThreads) void k_dt_partial(const double* __restrict__ ux,
-                                                           const double* __restrict__ uy,
-                                                           const double* __restrict__ hxxf,
-                                                           double hy, int nx, int ny, int rows,
-                                                           double* __restrict__ partial) {
-  dt_partial_body<NT>(ux, uy, hxxf, hy, nx, ny, rows, partial, blockIdx.x, blockIdx.y, gridDim.x);
+__global__ __launch_bounds__(kRedThreads) void k_dt(DtArgs a) {
+  dt_body<NT>(a, blockIdx.x, blockIdx.y);
 }
 
-// combine the limits (decide_dt.c:157-167)
-__device__ __forceinline__ void dt_final_body(const double* __restrict__ partial, int n, double cadv, double dif0,
-                                              double dif1, double dint, double* __restrict__ dt) {
-  __shared__ double sh[kRedThreads / 64];
-  double m = kDtMax;
-  // four running minima, so that the loads are in flight together (a
-  // minimum does not depend on the combination order)
-  double m1 = kDtMax, m2 = kDtMax, m3 = kDtMax;
-  const int s = (int)blockDim.x;
-  int k = threadIdx.x;
-  for (; k + 3 * s < n; k += 4 * s) {
-    m = fmin(m, partial[k]);
-    m1 = fmin(m1, partial[k + s]);
-    m2 = fmin(m2, partial[k + 2 * s]);
-    m3 = fmin(m3, partial[k + 3 * s]);
-  }
-  for (; k < n; k += s) m = fmin(m, partial[k]);
-  m = fmin(fmin(m, m1), fmin(m2, m3));
-  m = block_reduce<0>(m, sh);
-  if (threadIdx.x == 0) {
-    double r = m * cadv;
-    r = fmin(r, dif0);
-    r = fmin(r, dif1);
-    r = fmin(r, dint);
-    dt[0] = r;
-  }
-}
-
-__global__ void k_dt_final(const double* __restrict__ partial, int n, double cadv,
-                           double dif0, double dif1, double dint, double* __restrict__ dt) {
-  dt_final_body(partial, n, cadv, dif0, dif1, dint, dt);
-}
-
-// ensembles: one map entry (case, local block) per workgroup / one
-// workgroup per case
-__global__ __launch_bounds__(kRedThreads) void k_dt_partial_batch(const DtArgs* __restrict__ tab,
-                                                                 const uint2* __restrict__ map) {
+// ensembles: one map entry (case, local block) per workgroup
+__global__ __launch_bounds__(kRedThreads) void k_dt_batch(const DtArgs* __restrict__ tab,
+                                                         const uint2* __restrict__ map) {
   const uint2 m = map[blockIdx.x];
   const DtArgs& a = tab[m.x];
-  dt_partial_body<false>(a.ux, a.uy, a.hxxf, a.hy, a.nx, a.ny, a.rows, a.partial, (int)(m.y % a.gx), (int)(m.y / a.gx), a.gx);
-}
-
-__global__ __launch_bounds__(kRedThreads) void k_dt_final_batch(const DtArgs* __restrict__ tab) {
-  const DtArgs& a = tab[blockIdx.x];
-  dt_final_body(a.partial, a.nblk, a.cadv, a.dif0, a.dif1, a.dint, a.dt);
-}
-
-// the arguments of one case's decide_dt (dt limits from the host, as
-// compute_dt_device forms them)
-int dt_args(const domain_t* d, DomainCtx* c, const fluid_t* f, const interface_t* s, DtArgs* a) {
-  if (load_dt_coefs()) return 1;
-  const int nx = (int)c->nx, ny = (int)c->ny;
-  dt_limits(d, f, s, &a->dif0, &a->dif1, &a->dint);
-  int rows = 0, nblk = 0;
-  if (dt_grid(nx, ny, kRedSlots - 64, &rows, &nblk)) return 1;
-  a->ux = (const double*)f->ux.data;
-  a->uy = (const double*)f->uy.data;
-  a->hxxf = c->hxxf;
-  a->hy = c->hy;
-  a->cadv = options().cadv;
-  a->partial = c->red;
-  a->dt = c->dt_dev;
-  a->nx = nx;
-  a->ny = ny;
-  a->rows = rows;
-  a->gx = (int)cdiv(nx, kRedThreads);
-  a->nblk = a->gx * (int)cdiv(ny, rows);
-  return 0;
+  dt_body<false>(a, (int)(m.y % a.gx), (int)(m.y / a.gx));
 }
 
 // grid-only limits (decide_dt.c:79-130); host arithmetic identical to the
@@ -164,47 +139,45 @@ void dt_limits(const domain_t* d, const fluid_t* f, const interface_t* s, double
   *dint = di;
 }
 
-// Rows per partial-reduction workgroup: 16, doubled until the partial
-// minima fit `capacity` slots.  Fails (instead of looping on) a domain so
-// wide that one workgroup row alone needs more slots.
-int dt_grid(int nx, int ny, int capacity, int* rows, int* nblk) {
-  const long gx = cdiv(nx, kRedThreads);
-  int r = 16;
-  while (gx * cdiv(ny, r) > capacity && r < ny) r *= 2;
-  const long n = gx * cdiv(ny, r);
-  SBFS_REQUIRE(n <= capacity, "decide_dt: %d columns need %ld partial minima, more than the %d slots", nx, n,
-               capacity);
-  *rows = r;
-  *nblk = (int)n;
+// the arguments of one case's decide_dt, into `slot` and the pinned `host`.
+// Rows per workgroup: 4, doubled to at most 64 while the workgroups are more than
+// 2048, eight per CU (4096 x 8192: 90 us against 100 with at most 16 rows).
+int dt_args(const domain_t* d, const DomainCtx* c, const fluid_t* f, const interface_t* s, DtSlot* slot, double* host,
+            DtArgs* a) {
+  if (load_dt_coefs()) return 1;
+  dt_limits(d, f, s, &a->dif0, &a->dif1, &a->dint);
+  a->ux = (const double*)f->ux.data;
+  a->uy = (const double*)f->uy.data;
+  a->hxxf = c->hxxf;
+  a->hy = c->hy;
+  a->cadv = options().cadv;
+  a->slot = slot;
+  a->host = host;
+  a->nx = (int)c->nx;
+  a->ny = (int)c->ny;
+  a->gx = (int)cdiv(a->nx, kRedThreads);
+  SBFS_REQUIRE(a->gx <= kRedBlocks * 8, "decide_dt: %d columns need %d partial minima, more than the %d slots", a->nx,
+               a->gx, kRedBlocks * 8);
+  a->rows = 4;
+  while (a->gx * cdiv(a->ny, a->rows) > 2048 && a->rows < 64) a->rows *= 2;
+  a->nblk = a->gx * (int)cdiv(a->ny, a->rows);
   return 0;
 }
 
-// The dt reduction of one case into `partial` (at least dt_grid's nblk
-// doubles) and `dt_out` (one double), on the library stream.
-int dt_launch(const domain_t* d, const DomainCtx* c, const fluid_t* f, const interface_t* s,
-              int capacity, double* partial, double* dt_out) {
-  if (load_dt_coefs()) return 1;
-  const int nx = (int)c->nx, ny = (int)c->ny;
-  double dif0, dif1, dint;
-  dt_limits(d, f, s, &dif0, &dif1, &dint);
-  int rows = 0, nblk = 0;
-  if (dt_grid(nx, ny, capacity, &rows, &nblk)) return 1;
-  const dim3 grd(cdiv(nx, kRedThreads), cdiv(ny, rows));
-  SBFS_TIMED("k_dt_partial",
-             hipLaunchKernelGGL((stream_fields(nx, ny) ? k_dt_partial<true> : k_dt_partial<false>), grd,
-                                dim3(kRedThreads), 0, stream(),
-                                (const double*)f->ux.data, (const double*)f->uy.data, c->hxxf,
-                                c->hy, nx, ny, rows, partial));
-  SBFS_TIMED("k_dt_final",
-             hipLaunchKernelGGL(k_dt_final, dim3(1), dim3(kRedThreads), 0, stream(),
-                                (const double*)partial, nblk, options().cadv, dif0, dif1, dint,
-                                dt_out));
+int dt_launch(const DtArgs& a) {
+  const dim3 grd(a.gx, cdiv(a.ny, a.rows));
+  SBFS_TIMED("k_dt", hipLaunchKernelGGL((stream_fields(a.nx, a.ny) ? k_dt<true> : k_dt<false>), grd, dim3(kRedThreads),
+                                        0, stream(), a));
   return check_launch("decide_dt");
 }
 
+// dt into the domain's own slot, c->dt->dt, and, after the stream is
+// synchronised, *dt_host(c)
 int compute_dt_device(const domain_t* d, DomainCtx* c, const fluid_t* f,
                       const interface_t* s) {
-  return dt_launch(d, c, f, s, kRedSlots - 64, c->red, c->dt_dev);
+  DtArgs a;
+  if (dt_args(d, c, f, s, c->dt, dt_host(c), &a)) return 1;
+  return dt_launch(a);
 }
 
 // ---------------------------------------------------------------------------
@@ -323,9 +296,8 @@ int decide_dt(const domain_t* domain, const fluid_t* fluid, const interface_t* i
   if (check_array(domain, &fluid->ux, NA_UX, 8, "ux")) return 1;
   if (check_array(domain, &fluid->uy, NA_UY, 8, "uy")) return 1;
   if (compute_dt_device(domain, c, fluid, interface)) return 1;
-  SBFS_HIP(hipMemcpyAsync(c->host_pin, c->dt_dev, sizeof(double), hipMemcpyDeviceToHost, stream()));
   SBFS_HIP(hipStreamSynchronize(stream()));
-  *dt = c->host_pin[0];
+  *dt = *dt_host(c);
   return 0;
 }
 
