@@ -47,11 +47,16 @@ __device__ __forceinline__ void march_body(const MarchArgs& a, int bx, int by) {
   __shared__ double st[T_N][64];
   const int lane = threadIdx.x;
   const int nx = a.nx, ny = a.ny;
-  const int i0 = 1 + bx * kStrip;
+  // (the strip and rows are the same in every lane, but read from the dispatch
+  // order the compiler keeps them, and all that follows from them, in vector
+  // registers; said to be uniform they leave 26 of the FP64 bodies' 227 and 12
+  // of the mixed bodies' 168, whose row loop then spills nothing: at
+  // 2048 x 4096 mixed 215 -> 198 us, with the fold 287 -> 261 us)
+  const int i0 = __builtin_amdgcn_readfirstlane(1 + bx * kStrip);
   const int cl = i0 - 3;  // column held by lane 0
   const int c = cl + lane;
-  const int jb = 1 + by * a.band;
-  const int je = min(ny, jb + a.band - 1);
+  const int jb = __builtin_amdgcn_readfirstlane(1 + by * a.band);
+  const int je = __builtin_amdgcn_readfirstlane(min(ny, jb + a.band - 1));
   const bool c_vof = c >= 0 && c <= nx + 1;   // cells incl. wall ghosts
   const bool c_in = c >= 1 && c <= nx;        // interior cells
   const bool c_fx = c >= 1 && c <= nx + 1;    // x faces incl. walls
@@ -710,9 +715,9 @@ __global__ __launch_bounds__(1024) void k_march_order(const unsigned* __restrict
   }
 }
 
-// The FP64 bodies need about 230-250 VGPRs, two wavefronts per SIMD (three
+// The FP64 bodies need about 200 VGPRs, two wavefronts per SIMD (three
 // would spill dozens of registers to scratch, measured 1.4x slower).  The
-// FP32 bodies fit 168 VGPRs, three wavefronts per SIMD, which hides more of
+// FP32 bodies need 155 of 168 VGPRs, three wavefronts per SIMD, which hides more of
 // their latency (the folded variant 1.35x faster than at two).
 // The arguments arrive through a pointer to device memory, not by value:
 // held as kernel arguments, the ~50 uniform pointers and constants of
@@ -725,7 +730,7 @@ __device__ __forceinline__ bool march_unit(const MarchArgs& a, int& bx, int& by)
   bx = blockIdx.x;
   by = blockIdx.y;
   if (a.order) {
-    const unsigned u = a.order[blockIdx.x];
+    const unsigned u = (unsigned)__builtin_amdgcn_readfirstlane((int)a.order[blockIdx.x]);
     if (u >= (unsigned)march_units(a.nx, a.ny, a.band)) return false;
     const int strips = march_strips(a.nx);
     bx = (int)u % strips;
