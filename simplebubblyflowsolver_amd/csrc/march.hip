@@ -33,18 +33,35 @@
 
 namespace sbfs {
 
+// LDS of one wavefront: the column tables, and the older rows that the folded
+// FP32 body keeps there (it has no VGPRs left for them; each lane reads back
+// only what it wrote, so no barrier is needed).  The FP64 body has: with them
+// in LDS its folded kernel took 355 us instead of 352 at 2048 x 4096.
+enum { RG_QUXS, RG_CYCUYS, RG_D1X, RG_CGY, RG_PSM1, RG_PM1, RG_DNM1, RG_N };
+template <bool LR>
+struct MarchLds {
+  double st[T_N][64];
+  double rings[LR ? RG_N : 1][64];
+};
+template <typename R, bool CORR>
+constexpr bool kLdsRings = CORR && std::is_same<R, float>::value;
+
 // R = double: the plain FP64 step.  R = float: the stencils of the
 // interface (gradients, normals, curvature, THINC and mass fluxes) and of the
 // momentum sources (viscosities, stresses, advection, surface tension,
 // buoyancy) in FP32; the vof update, the density-weighted velocity update,
 // the pressure gradient and the Poisson right-hand side stay FP64.
 // (bx, by): the strip and band of this wavefront
+// IN: every lane of the strip holds an interior cell that touches no wall
+// (march_inner): only the interface and the strip's output columns mask lanes
 // NT: the FP64 bodies store their output rows streaming (see ST below)
-template <typename R, bool CORR, bool NT = false>
-__device__ __forceinline__ void march_body(const MarchArgs& a, int bx, int by) {
+template <typename R, bool CORR, bool NT, bool IN>
+__device__ __forceinline__ void march_body(const MarchArgs& a, int bx, int by,
+                                           MarchLds<kLdsRings<R, CORR>>& lds) {
   using A = Arith<R>;
   using V3 = V3R<R>;
-  __shared__ double st[T_N][64];
+  auto& st = lds.st;
+  auto& rings = lds.rings;
   const int lane = threadIdx.x;
   const int nx = a.nx, ny = a.ny;
   // (the strip and rows are the same in every lane, but read from the dispatch
@@ -57,10 +74,12 @@ __device__ __forceinline__ void march_body(const MarchArgs& a, int bx, int by) {
   const int c = cl + lane;
   const int jb = __builtin_amdgcn_readfirstlane(1 + by * a.band);
   const int je = __builtin_amdgcn_readfirstlane(min(ny, jb + a.band - 1));
-  const bool c_vof = c >= 0 && c <= nx + 1;   // cells incl. wall ghosts
-  const bool c_in = c >= 1 && c <= nx;        // interior cells
-  const bool c_fx = c >= 1 && c <= nx + 1;    // x faces incl. walls
-  const bool c_out = c >= i0 && c < i0 + kStrip && c <= nx;
+  const bool c_vof = IN || (c >= 0 && c <= nx + 1);   // cells incl. wall ghosts
+  const bool c_in = IN || (c >= 1 && c <= nx);        // interior cells
+  const bool c_fx = IN || (c >= 1 && c <= nx + 1);    // x faces incl. walls
+  const bool c_ux = IN || (c >= 2 && c <= nx);        // x faces between interior cells
+  const bool c_first = !IN && c == 1, c_last = !IN && c == nx;
+  const bool c_out = c >= i0 && c < i0 + kStrip && (IN || c <= nx);
   const int cc = c < 0 ? 0 : (c > nx + 1 ? nx + 1 : c);
   {
     const double* tabs[T_N] = {a.cf.rhf, a.cf.rhc, a.cf.rjf, a.cf.rjc, a.cf.qf, a.cf.qc, a.cf.eqf,
@@ -68,13 +87,7 @@ __device__ __forceinline__ void march_body(const MarchArgs& a, int bx, int by) {
 #pragma unroll
     for (int t = 0; t < T_N; t++) st[t][lane] = tabs[t][cc];
   }
-  // The folded projection needs more VGPRs than the plain body has left, so
-  // that variant keeps its older rows of the Poisson right-hand side, the
-  // potential, the pressure and the new density in LDS instead (each lane
-  // reads back only what it wrote, so no barrier is needed).
-  constexpr bool LR = CORR;
-  enum { RG_QUXS, RG_CYCUYS, RG_D1X, RG_CGY, RG_PSM1, RG_PM1, RG_DNM1, RG_N };
-  __shared__ double rings[LR ? RG_N : 1][64];
+  constexpr bool LR = kLdsRings<R, CORR>;
   if (LR)
     for (int k = 0; k < RG_N; k++) rings[k][lane] = 0.;
   __syncthreads();
@@ -139,8 +152,8 @@ __device__ __forceinline__ void march_body(const MarchArgs& a, int bx, int by) {
   // viscosity at x face c from the vof on its two sides (viscosity.c:37-53)
   auto VISUX = [&](int col, R vl, R vr) {
     R v;
-    if (col == 1) v = vl;
-    else if (col == nx + 1) v = vr;
+    if (!IN && col == 1) v = vl;
+    else if (!IN && col == nx + 1) v = vr;
     else v = R(0.5) * vl + R(0.5) * vr;
     return mixr<R>(a.visr, a.vlo, a.vhi, v);
   };
@@ -224,7 +237,7 @@ __device__ __forceinline__ void march_body(const MarchArgs& a, int bx, int by) {
     if (has_b && c_in) {
       bv = AT(ci_row(a.srcb_vof, jw));
       if (s_ >= jb) by = msrc(a.srcb_uy, ci_row, jw);
-      if (s_ >= jb && s_ <= je && c >= 2) bx = msrc(a.srcb_ux, fx_row, jw);
+      if (s_ >= jb && s_ <= je && (IN || c >= 2)) bx = msrc(a.srcb_ux, fx_row, jw);
     }
   };
   double nsbv;
@@ -349,7 +362,7 @@ __device__ __forceinline__ void march_body(const MarchArgs& a, int bx, int by) {
       R mf = 0;
       if (c_fx) {
         const R vel = rux0;
-        if (c != 1 && c != nx + 1) {
+        if (IN || (c != 1 && c != nx + 1)) {
           const bool up = vel < R(0);
           const double v = up ? v0 : vl;
           const V3 n = up ? V3{n0x, n0y, n0z} : V3{nlx, nly, nlz};
@@ -366,7 +379,7 @@ __device__ __forceinline__ void march_body(const MarchArgs& a, int bx, int by) {
       R f = 0, mf = 0;
       if (c_vof) {
         const R vel = ruyp1;
-        if (c != 0 && c != nx + 1) {
+        if (IN || (c != 0 && c != nx + 1)) {
           const bool up = vel < R(0);
           const double v = up ? vp1 : v0;
           const V3 n = up ? V3{n1x, n1y, n1z} : V3{n0x, n0y, n0z};
@@ -479,7 +492,7 @@ __device__ __forceinline__ void march_body(const MarchArgs& a, int bx, int by) {
         const double p0l = from_left(p0);
         const R k0l = A::left(k0);
         // -- predicted ux, row s (predict/ux.c, force.c) -----------------------
-        if (c >= 2 && c <= nx) {
+        if (c_ux) {
           R s_ = 0;
           s_ -= SB(T_RJF) * (-qxl + qx);
           s_ -= SB(T_RJF) * (-qy_ux + qy_ux_new);
@@ -545,29 +558,29 @@ __device__ __forceinline__ void march_body(const MarchArgs& a, int bx, int by) {
         auto rc = [&](double* f, int j) { return cc_row(f, j); };
         auto rx = [&](double* f, int j) { return xf_row(f, j); };
         put(a.vofn, 2, rv, vn0);
-        if (c == 1) put_at(a.vofn, 2, rv, -1, 0.);
-        if (c == nx) put_at(a.vofn, 2, rv, 1, 0.);
+        if (c_first) put_at(a.vofn, 2, rv, -1, 0.);
+        if (c_last) put_at(a.vofn, 2, rv, 1, 0.);
         if (a.srca_vof) ST(ci_row(a.srca_vof, s), src);
-        put(a.uxs, 1, rx, c == 1 ? 0. : uxs);
-        if (c == nx) put_at(a.uxs, 1, rx, 1, 0.);
+        put(a.uxs, 1, rx, c_first ? 0. : uxs);
+        if (c_last) put_at(a.uxs, 1, rx, 1, 0.);
         put(a.uys, 1, rc, uys);
-        if (c == 1) put_at(a.uys, 1, rc, -1, kUyXm);
-        if (c == nx) put_at(a.uys, 1, rc, 1, kUyXp);
+        if (c_first) put_at(a.uys, 1, rc, -1, kUyXm);
+        if (c_last) put_at(a.uys, 1, rc, 1, kUyXp);
         if (a.den1) {
           const double dg = DEN(0.);
           put(a.den1, 1, rc, dn0);
-          if (c == 1) put_at(a.den1, 1, rc, -1, dg);
-          if (c == nx) put_at(a.den1, 1, rc, 1, dg);
+          if (c_first) put_at(a.den1, 1, rc, -1, dg);
+          if (c_last) put_at(a.den1, 1, rc, 1, dg);
         }
         if (a.txy) {
           put(a.txy, 1, rx, double(txy_prev));
-          if (c == nx) put_at(a.txy, 1, rx, 1, txy0r);
+          if (c_last) put_at(a.txy, 1, rx, 1, txy0r);
         }
         if (CORR && a.p_out) {
           // the previous stage's updated pressure, with its Neumann ghosts
           put(a.p_out, 1, rc, p0);
-          if (c == 1) put_at(a.p_out, 1, rc, -1, p0);
-          if (c == nx) put_at(a.p_out, 1, rc, 1, p0);
+          if (c_first) put_at(a.p_out, 1, rc, -1, p0);
+          if (c_last) put_at(a.p_out, 1, rc, 1, p0);
         }
       }
     }
@@ -618,7 +631,7 @@ __device__ __forceinline__ void march_body(const MarchArgs& a, int bx, int by) {
       const double nps_l = from_left(nps), npo_l = from_left(npo);
       {
         double u = 0.;
-        if (c >= 2 && c <= nx) {
+        if (c_ux) {
           u = nux;
           u -= per_h(pcx0) * (-nps_l + nps);
           const double d = 0.5 * dbl + 0.5 * db;
@@ -628,8 +641,8 @@ __device__ __forceinline__ void march_body(const MarchArgs& a, int bx, int by) {
       }
       {
         double u = 0.;
-        if (c == 0) u = kUyXm;
-        else if (c == nx + 1) u = kUyXp;
+        if (!IN && c == 0) u = kUyXm;
+        else if (!IN && c == nx + 1) u = kUyXp;
         else if (c_in) {
           u = nuy;
           u -= pcy * (-psp1 + nps);
@@ -715,7 +728,7 @@ __global__ __launch_bounds__(1024) void k_march_order(const unsigned* __restrict
   }
 }
 
-// The FP64 bodies need about 200 VGPRs, two wavefronts per SIMD (three
+// The FP64 bodies need 199 to 222 VGPRs, two wavefronts per SIMD (three
 // would spill dozens of registers to scratch, measured 1.4x slower).  The
 // FP32 bodies need 155 of 168 VGPRs, three wavefronts per SIMD, which hides more of
 // their latency (the folded variant 1.35x faster than at two).
@@ -738,19 +751,35 @@ __device__ __forceinline__ bool march_unit(const MarchArgs& a, int& bx, int& by)
   }
   return true;
 }
+// Whether every lane of strip bx holds an interior cell away from the walls
+// (all strips but the first and the last one or two): in FP64 those run the body
+// without the walls' lane masks.  In the masked body about 170 exec-mask blocks
+// with their branches interrupt a row step, which every strip paid for the few
+// at the walls; without them k_march takes 264 us instead of 283 at 2048 x 4096
+// and 1102 instead of 1175 at 4096 x 8192, with the fold 338 instead of 347 and
+// 1414 instead of 1450.  The FP32 bodies, which wait for memory more than they
+// compute, got slower (2048 x 4096: 206 us against 198, with the fold 273 against 261)
+// and keep the one masked body.
+__device__ __forceinline__ bool march_inner(int nx, int bx) { return bx >= 1 && 1 + bx * kStrip + 60 <= nx; }
+template <typename R, bool CORR, bool NT>
+__device__ __forceinline__ void march_strip(const MarchArgs& a, int bx, int by) {
+  __shared__ MarchLds<kLdsRings<R, CORR>> lds;
+  if (std::is_same<R, double>::value && march_inner(a.nx, bx)) march_body<R, CORR, NT, true>(a, bx, by, lds);
+  else march_body<R, CORR, NT, false>(a, bx, by, lds);
+}
 #define SBFS_MARCH_KERNEL(name, R, CORR, WAVES)                                            \
   __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WAVES))) void name( \
       const MarchArgs* __restrict__ args) {                                               \
     const MarchArgs& a = *args;                                                           \
     int bx, by;                                                                           \
-    if (march_unit(a, bx, by)) march_body<R, CORR>(a, bx, by);                            \
+    if (march_unit(a, bx, by)) march_strip<R, CORR, false>(a, bx, by);                    \
   }                                                                                       \
   __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WAVES))) void name##_batch( \
       const MarchArgs* __restrict__ tab, const uint2* __restrict__ map) {                \
     const uint2 m = map[blockIdx.x];                                                      \
     const MarchArgs& a = tab[m.x];                                                        \
     const int strips = (a.nx + kStrip - 1) / kStrip;                                      \
-    march_body<R, CORR>(a, (int)m.y % strips, (int)m.y / strips);                         \
+    march_strip<R, CORR, false>(a, (int)m.y % strips, (int)m.y / strips);                 \
   }
 SBFS_MARCH_KERNEL(k_march, double, false, SBFS_FP64_WAVES)
 SBFS_MARCH_KERNEL(k_march_corr, double, true, SBFS_FP64_WAVES)
@@ -764,7 +793,7 @@ SBFS_MARCH_KERNEL(k_march_mixed_corr, float, true, SBFS_MIXED_WAVES)
       const MarchArgs* __restrict__ args) {                                                      \
     const MarchArgs& a = *args;                                                                  \
     int bx, by;                                                                                  \
-    if (march_unit(a, bx, by)) march_body<double, CORR, true>(a, bx, by);                        \
+    if (march_unit(a, bx, by)) march_strip<double, CORR, true>(a, bx, by);                       \
   }
 SBFS_MARCH_NT_KERNEL(k_march_nt, false)
 SBFS_MARCH_NT_KERNEL(k_march_corr_nt, true)
