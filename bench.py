@@ -66,6 +66,7 @@ BYTES_PER_CELL = {
     "k_force": 40, "k_fluxx": 48, "k_fluxy": 48, "k_vof_advance": 48, "k_mass_flux": 48,
     "k_stress": 56, "k_rhs_ux": 80, "k_rhs_uy": 72, "k_predict_ux": 56, "k_predict_uy": 56,
     "k_dct2_rhs": 40, "k_tdm_sequential": 16, "k_part_reduce": 16, "k_part_conv": 0,
+    "k_part_solve": 16, "k_tdm_columns": 16,
     "k_dct3_psi": 16, "k_correct_ux": 40, "k_correct_uy": 40,
     "k_update_p": 24, "k_dt": 16,
     # fused path
@@ -74,6 +75,7 @@ BYTES_PER_CELL = {
     # 8 fewer in stages 1 and 2)
     "k_march": 12 * 8, "k_march_mixed": 12 * 8 - 8, "k_dct2_rows": 16,
     "k_post": 72, "k_march_corr": 16 * 8, "k_march_mixed_corr": 16 * 8 - 12,
+    "k_tile": 12 * 8, "k_tile_mixed": 12 * 8 - 8, "k_tile_corr": 16 * 8, "k_tile_mixed_corr": 16 * 8 - 12,
     # learned curvature: the stage-0 gate reads the vof field
     "k_curv_gate": 8,
 }

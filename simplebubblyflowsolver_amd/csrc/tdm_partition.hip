@@ -209,6 +209,69 @@ __global__ __launch_bounds__(256) void k_part_conv(const double* __restrict__ q,
   }
 }
 
+// T1 and T2 in one launch, for the solves of part_fused: a workgroup holds all
+// P chunks of 2^ms modes, a thread one of them, so the chunks' ends, the
+// reduced right-hand side and the inverse columns (twice over, so that the
+// window needs no wrap) never leave LDS.  Operations and their order are those
+// of k_part_reduce and k_part_conv.  Bound by latency: the VGPRs of two
+// wavefronts per SIMD let a thread issue all loads of its chunk at once (held
+// to 128 of them the 512 x 1024 solve took 13.7 us instead of 3.4).
+constexpr int kPartThreads = 128;
+template <int L>
+__global__ __launch_bounds__(kPartThreads) __attribute__((amdgpu_waves_per_eu(1, 2))) void k_part_solve(
+    double* __restrict__ q, const double* __restrict__ tab, const double* __restrict__ htab, double* __restrict__ X,
+    int nx, int P, double a, int pin_mode0, int ms) {
+  constexpr int K = L - 1;
+  extern __shared__ double lds[];
+  const int group = xcd_group((int)blockIdx.x, (int)gridDim.x);
+  const int ch = (int)threadIdx.x >> ms, tm = (int)threadIdx.x & ((1 << ms) - 1), mo = (group << ms) + tm;
+  const bool act = ch < P;
+  double* R = lds;                // [P][2^ms] reduced right-hand side
+  double* H = R + (P << ms);      // [2 P][2^ms] inverse columns
+  double* F = H + (2 * P << ms);  // [P][2^ms] first values, then the result
+  const int at = (ch << ms) + tm;
+  double sep = 0., first = 0., last = 0.;
+  if (act) {
+    sep = q[(size_t)(ch * L + K) * nx + mo];
+    const double h = htab[(size_t)ch * nx + mo];
+    H[at] = h;
+    H[at + (P << ms)] = h;
+    chunk_reduce<K, false>(q, nx, mo, ch * L, tab, tab + (size_t)K * nx, a, first, last, nullptr);
+    F[at] = first;
+  }
+  __syncthreads();
+  if (act) R[at] = (sep - a * last) - a * F[ch + 1 < P ? at + (1 << ms) : tm];
+  __syncthreads();
+  double acc = 0.;
+  if (act) {
+    const double *h = H + at + (P << ms), *r = R + tm;  // h[(ch - k) mod P], R_k
+#pragma unroll 8
+    for (int k = 0; k < P; k++) acc += h[-(k << ms)] * r[k << ms];
+  }
+  if (pin_mode0 && group == 0) {
+    if (act) F[at] = acc;
+    __syncthreads();
+    if (mo == 0) acc = acc - F[(P - 1) << ms];
+  }
+  if (act) X[(size_t)ch * nx + mo] = acc;
+}
+
+// k_part_solve's modes per workgroup, as a power of two: four, or as many as
+// fill a wavefront with P chunks each
+static int part_modes(int nx, int P) {
+  int ms = P <= 4 ? 4 : P <= 8 ? 3 : 2;
+  while ((1 << ms) > nx) ms--;
+  return ms;
+}
+// One launch while it is bound by latency and a workgroup holds the chunks.  With
+// 32768 chunks in all a step gains (1024 x 1024 mixed 299 -> 291 us, 512 x 1024
+// 236 -> 228, 64 x 128 131 -> 118), with 65536 the short row segments of four
+// modes cost as much as the launch (2048 x 1024 429 -> 432, 4096 x 512 equal), and
+// so does a workgroup of 64 chunks (512 x 2048 368 -> 370).
+static bool part_fused(int nx, int P, int L) {
+  return L <= 32 && (P << part_modes(nx, P)) <= kPartThreads && (long)nx * P <= 32768;
+}
+
 // per-mode tables (same arithmetic as the oracle's chunk tables)
 static void host_thomas(int K, const double* inv, const double* v, double a, const double* f,
                         double* g) {
@@ -311,6 +374,16 @@ int partition_setup(PoissonPlan* p, const domain_t* d, int L) {
 template <int L>
 static void part_launch(PoissonPlan* p, double a, int pin) {
   const int nx = p->nx, P = p->P;
+  if constexpr (L <= 32) {
+    if (part_fused(nx, P, L)) {
+      const int ms = part_modes(nx, P);
+      SBFS_TIMED("k_part_solve",
+                 hipLaunchKernelGGL(k_part_solve<L>, dim3(nx >> ms), dim3(cdiv(P << ms, 64) * 64),
+                                    sizeof(double) * 4 * ((size_t)P << ms), stream(), p->buf, p->ptab, p->htab, p->X,
+                                    nx, P, a, pin, ms));
+      return;
+    }
+  }
   const dim3 blk(64, 4), grd(cdiv(nx, 64), cdiv(P, 4));
   SBFS_TIMED("k_part_reduce",
              hipLaunchKernelGGL(k_part_reduce<L>, grd, blk, 0, stream(), p->buf, p->ptab, p->gfl,
