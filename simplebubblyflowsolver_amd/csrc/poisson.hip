@@ -247,9 +247,9 @@ __device__ __forceinline__ void st_row(T* p, T v) {
 // the unit's rows in LDS: row rr at lds + rr PM, doubles through zd().
 // Rows past the last (rr >= nrows >= 1) load the last row again, so every
 // load is unconditional and all are in flight before the first LDS write.
-template <int LOG, typename Src>
+template <int FORM, typename Src>
 __device__ __forceinline__ void rows_to_lds(double2* lds, int lane, int nrows, Src src) {
-  using F = WaveFft<LOG>;
+  using F = WaveFft<FORM>;
   constexpr int H = F::N / 2;  // double2 per row
   if constexpr (F::R * H >= F::U) {
     constexpr int PER = F::R * H / F::U;
@@ -271,19 +271,28 @@ __device__ __forceinline__ void rows_to_lds(double2* lds, int lane, int nrows, S
 }
 
 // (the unit's LDS rows at `lds`, its thread `lane` in [0, U))
-template <int LOG, bool NT>
+template <int FORM, bool NT>
 __device__ __forceinline__ void dct2_wave(const double* __restrict__ in, double* __restrict__ out, int rows,
                                           int row0, const double2* __restrict__ tw,
                                           const double2* __restrict__ t1, const double2* __restrict__ t2,
                                           double2* lds, int lane) {
-  using F = WaveFft<LOG>;
+  using F = WaveFft<FORM>;
   constexpr int M = F::M, N = F::N, G = F::G;
   const int rg = lane / G, lt = lane % G;
   const int nrows = min(F::R, rows - row0);
   if (nrows <= 0) return;  // a second unit past the last row (one wavefront, no barrier)
-  const auto tw0 = pass_tw<LOG, 0>(lt, tw);
+  const auto tw0 = pass_tw<FORM, 0>(lt, tw);
+  // (the short form's post-twiddles, loaded before the row like its others)
+  double2 post1[F::SHORT ? M / G + 1 : 1], post2[F::SHORT ? M / G + 1 : 1];
+  if constexpr (F::SHORT) {
+#pragma unroll
+    for (int i = 0; i <= M / G; i++) {
+      post1[i] = t1[min(lt + i * G, M)];
+      post2[i] = t2[min(lt + i * G, M)];
+    }
+  }
   const double2* src = (const double2*)(in + (size_t)row0 * N);
-  rows_to_lds<LOG>(lds, lane, nrows, [src](int rr, int h) { return ld_row<NT>(src + rr * (N / 2) + h); });
+  rows_to_lds<FORM>(lds, lane, nrows, [src](int rr, int h) { return ld_row<NT>(src + rr * (N / 2) + h); });
   F::sync();
   double2* Z = lds + rg * F::PM;
   // v[k] = x[2k], v[n-1-k] = x[2k+1]; z[k] = v[2k] + i v[2k+1]
@@ -293,13 +302,14 @@ __device__ __forceinline__ void dct2_wave(const double* __restrict__ in, double*
     const double vo = (o < M) ? zd(Z, 2 * o) : zd(Z, 2 * (N - 1 - o) + 1);
     return make_double2(ve, vo);
   };
-  wave_fft<LOG>(Z, lt, tw, ld0, tw0);
+  wave_fft<FORM>(Z, lt, tw, ld0, tw0);
   if (rg >= nrows) return;
   double* dst = out + (size_t)(row0 + rg) * N;
 #pragma unroll
   for (int i = 0; i <= M / G; i++) {
     const int k = lt + i * G;
     if (k > M) break;
+    const double2 w1 = F::SHORT ? post1[i] : t1[k], w2 = F::SHORT ? post2[i] : t2[k];
     const int kk = (k == M) ? 0 : k;
     const int kr = (k == 0) ? 0 : M - k;
     const double2 za = Z[fpad(kk)], zb = Z[fpad(kr)];
@@ -308,9 +318,9 @@ __device__ __forceinline__ void dct2_wave(const double* __restrict__ in, double*
     const double er = (ar + br) * 0.5, ei = (ai + bi) * 0.5;
     const double dr = ar - br, di = ai - bi;
     const double2 od = make_double2(di * 0.5, -(dr * 0.5));
-    const double2 tt = wmul(od, t1[k]);
+    const double2 tt = wmul(od, w1);
     const double2 vv = make_double2(er + tt.x, ei + tt.y);
-    const double2 w = wmul(vv, t2[k]);
+    const double2 w = wmul(vv, w2);
     st_row<NT>(dst + k, 2. * w.x);
     if (k != 0 && k != M) st_row<NT>(dst + (N - k), -2. * w.y);
   }
@@ -343,12 +353,12 @@ struct ModeSrc {
 // last row (the separator itself) are the same for every
 // lane; with several, the loads are unconditional (a chunk's last row
 // reads spike row 0, whose product it discards) and the value a select.
-template <int LOG, bool NT>
+template <int FORM, bool NT>
 __device__ __forceinline__ void expanded_to_lds(double2* lds, int lane, int nrows, const ModeSrc& src, int row0) {
-  using F = WaveFft<LOG>;
+  using F = WaveFft<FORM>;
   constexpr int H = F::N / 2;  // double2 per row
   static_assert(F::R * H >= F::U, "every lane loads at least one point");
-  constexpr int PER = F::R * H / F::U, GMAX = LOG >= 11 ? 8 : 4, GRP = PER < GMAX ? PER : GMAX;
+  constexpr int PER = F::R * H / F::U, GMAX = F::LOG >= 11 ? 8 : 4, GRP = PER < GMAX ? PER : GMAX;
   static_assert(PER % GRP == 0, "groups of points");
   const int nx = src.nx, sh = 31 - __clz(src.L);
   auto row = [&](int i) { return F::R == 1 ? row0 : row0 + min((lane + i * F::U) / H, nrows - 1); };
@@ -400,16 +410,16 @@ __device__ __forceinline__ void expanded_to_lds(double2* lds, int lane, int nrow
 // psi[1] rows j = row + 1 with the Neumann x ghosts and the periodic y halo
 // (compute_potential.c:365-380, src/fluid/boundary/psi.c; out must be
 // 16-byte aligned); otherwise plain rows of N
-template <int LOG, bool PSI, int AHEAD, bool NT>
+template <int FORM, bool PSI, int AHEAD, bool NT>
 __device__ __forceinline__ void dct3_wave(const ModeSrc& src, int rows, int row0, const double2* __restrict__ tw,
                                           const double2* __restrict__ t1, const double2* __restrict__ t2,
                                           double* __restrict__ out, double2* lds, int lane) {
-  using F = WaveFft<LOG>;
+  using F = WaveFft<FORM>;
   constexpr int M = F::M, N = F::N, G = F::G;
   const int rg = lane / G, lt = lane % G;
   const int nrows = min(F::R, rows - row0);
   if (nrows <= 0) return;  // a second unit past the last row (one wavefront, no barrier)
-  const auto tw0 = pass_tw<LOG, 0>(lt, tw);
+  const auto tw0 = pass_tw<FORM, 0>(lt, tw);
   // the pre-twiddle's factors of k and M - k for iteration i (k = lt + i G,
   // the last iteration only for k = M / 2): with AHEAD > 0 the first AHEAD
   // iterations' are loaded before the row and the others AHEAD iterations
@@ -428,9 +438,9 @@ __device__ __forceinline__ void dct3_wave(const ModeSrc& src, int rows, int row0
 #pragma unroll
   for (int i = 0; i < AHEAD; i++) fetch(i);
   if (src.L == 0)
-    rows_to_lds<LOG>(lds, lane, nrows, [&src, row0](int rr, int h) { return src.solved(row0 + rr, h); });
+    rows_to_lds<FORM>(lds, lane, nrows, [&src, row0](int rr, int h) { return src.solved(row0 + rr, h); });
   else
-    expanded_to_lds<LOG, NT>(lds, lane, nrows, src, row0);
+    expanded_to_lds<FORM, NT>(lds, lane, nrows, src, row0);
   F::sync();
   double2* Z = lds + rg * F::PM;
   // pre-twiddle in place: the values of k and M - k (0 <= k <= M/2) need
@@ -479,7 +489,7 @@ __device__ __forceinline__ void dct3_wave(const ModeSrc& src, int rows, int row0
     if (2 * j < M) return make_double2(zd(Z, j), zd(Z, M - j));
     return make_double2(zd(Z, 2 * M - j), zd(Z, M + j));
   };
-  wave_fft<LOG>(Z, lt, tw, ld0, tw0);
+  wave_fft<FORM>(Z, lt, tw, ld0, tw0);
   // y[2x] (x < M) and y[2(N-1-x)+1] (x >= M) take z[x/2].x for even x and
   // -z[x/2].y for odd x
   if (rg >= nrows) return;
@@ -522,26 +532,26 @@ __device__ __forceinline__ void dct3_wave(const ModeSrc& src, int rows, int row0
 // hoisting every load
 #define SBFS_ROWS_ATTR(LG) __launch_bounds__(wave_fft_u(LG)) __attribute__((amdgpu_waves_per_eu(2)))
 
-template <int LOG, bool NT>
-__global__ SBFS_ROWS_ATTR(LOG) void k_dct2_rows(const double* __restrict__ in, double* __restrict__ out, int rows,
+template <int FORM, bool NT>
+__global__ SBFS_ROWS_ATTR(FORM) void k_dct2_rows(const double* __restrict__ in, double* __restrict__ out, int rows,
                                                 const double2* __restrict__ tw, const double2* __restrict__ t1,
                                                 const double2* __restrict__ t2) {
   extern __shared__ double2 lds[];
-  dct2_wave<LOG, NT>(in, out, rows, (int)blockIdx.x * WaveFft<LOG>::R, tw, t1, t2, lds, (int)threadIdx.x);
+  dct2_wave<FORM, NT>(in, out, rows, (int)blockIdx.x * WaveFft<FORM>::R, tw, t1, t2, lds, (int)threadIdx.x);
 }
 
-template <int LOG>
-__global__ SBFS_ROWS_ATTR(LOG) void k_dct3_rows(const double* __restrict__ in, double* __restrict__ out, int rows,
+template <int FORM>
+__global__ SBFS_ROWS_ATTR(FORM) void k_dct3_rows(const double* __restrict__ in, double* __restrict__ out, int rows,
                                                 const double2* __restrict__ tw, const double2* __restrict__ t1,
                                                 const double2* __restrict__ t2) {
-  constexpr int N = WaveFft<LOG>::N;
+  constexpr int N = WaveFft<FORM>::N;
   extern __shared__ double2 lds[];
   const ModeSrc src{in, nullptr, nullptr, nullptr, N, 0, 0};
-  dct3_wave<LOG, false, 1, false>(src, rows, (int)blockIdx.x * WaveFft<LOG>::R, tw, t1, t2, out, lds, (int)threadIdx.x);
+  dct3_wave<FORM, false, 1, false>(src, rows, (int)blockIdx.x * WaveFft<FORM>::R, tw, t1, t2, out, lds, (int)threadIdx.x);
 }
 
-template <int LOG, bool NT>
-__global__ SBFS_ROWS_ATTR(LOG) void k_dct3_psi(ModeSrc src, double* __restrict__ psi, int ny,
+template <int FORM, bool NT>
+__global__ SBFS_ROWS_ATTR(FORM) void k_dct3_psi(ModeSrc src, double* __restrict__ psi, int ny,
                                                const double2* __restrict__ tw, const double2* __restrict__ t1,
                                                const double2* __restrict__ t2) {
   extern __shared__ double2 lds[];
@@ -552,25 +562,40 @@ __global__ SBFS_ROWS_ATTR(LOG) void k_dct3_psi(ModeSrc src, double* __restrict__
   // separators of its own chunks.
   int unit;
   const int n = (int)gridDim.x, b = (int)blockIdx.x;
-  if (WaveFft<LOG>::R == 1 && src.L >= 4 && (src.P & 1) == 0 && (n & 7) == 0) {
+  if (WaveFft<FORM>::R == 1 && src.L >= 4 && (src.P & 1) == 0 && (n & 7) == 0) {
     const int x = b & 7, i = b >> 3, kq = src.L / 4;
     unit = ((x >> 2) * (src.P / 2) + i / kq) * src.L + (x & 3) * kq + i % kq;
   } else {
     unit = xcd_group(b, n);
   }
-  dct3_wave<LOG, true, 1, NT>(src, ny, unit * WaveFft<LOG>::R, tw, t1, t2, psi, lds, (int)threadIdx.x);
+  dct3_wave<FORM, true, WaveFft<FORM>::SHORT ? 3 : 1, NT>(src, ny, unit * WaveFft<FORM>::R, tw, t1, t2, psi, lds, (int)threadIdx.x);
 }
 
-#define SBFS_LOG_CASES(X) \
-  X(0) X(1) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(11)
+// the forms that row_form gives
+#define SBFS_FORM_CASES(X) \
+  X(0) X(1) X(kShort + 2) X(kShort + 3) X(kShort + 4) X(kShort + 5) X(kShort + 6) X(kShort + 7) X(kShort + 8) \
+  X(kShort + 9) X(10) X(kShort + 10) X(11)
 
 static int ilog2(int m) { return 31 - __builtin_clz((unsigned)m); }
 
-// rows, threads and LDS bytes of one unit of the row transforms for m
-// complex points
-int wave_rows(int m) { return wave_fft_r(ilog2(m)); }
-int wave_unit(int m) { return wave_fft_u(ilog2(m)); }
-size_t wave_lds(int m) { return wave_fft_lds(ilog2(m)); }
+// Form of a transform of `rows` rows of m complex points (rowfft.hpp): the
+// short one up to 1024 columns, where it is the faster at every row count (DCT-III
+// and DCT-II at 64 x 128 10.9 -> 6.8 and 7.5 -> 6.2 us, 512 x 1024 12.8 -> 8.8 and
+// 9.3 -> 6.7, 1024 x 2048 21.4 -> 18.0 and 15.9 -> 12.3, 1024 x 8192 48.4 -> 46.4
+// and 39.0 -> 36.7), and at 2048 columns up to 1024 rows (19.9 -> 18.4 and
+// 16.0 -> 12.7; with 2048 rows 27.2 -> 29.7 and 20.8 -> 21.8).
+static int row_form(int m, int rows) {
+  const int lg = ilog2(m);
+  return lg >= 2 && (lg <= 9 || (lg == 10 && rows <= 1024)) ? lg + kShort : lg;
+}
+// (an ensemble's: the units of its workgroups have at most 128 threads)
+static __host__ __device__ int row_form_batch(int lg) { return lg >= 2 && lg <= 9 ? lg + kShort : lg; }
+
+// rows, threads and LDS bytes of one unit of an ensemble's row transforms for
+// m complex points
+int wave_rows(int m) { return wave_fft_r(row_form_batch(ilog2(m))); }
+int wave_unit(int m) { return wave_fft_u(row_form_batch(ilog2(m))); }
+size_t wave_lds(int m) { return wave_fft_lds(row_form_batch(ilog2(m))); }
 
 // ---------------------------------------------------------------------------
 // tridiagonal solves, reference order: one Thomas + Sherman-Morrison chain
@@ -828,6 +853,9 @@ static int sequential_solve(PoissonPlan* p, double l, int pin) {
   return check_launch("poisson: tridiagonal");
 }
 
+#define SBFS_BATCH_CASES(X) \
+  X(0) X(1) X(kShort + 2) X(kShort + 3) X(kShort + 4) X(kShort + 5) X(kShort + 6) X(kShort + 7) X(kShort + 8) \
+  X(kShort + 9) X(10) X(11)
 // ensembles: one map entry (case, group of rows or of 64 modes) per
 // workgroup; the row transforms switch on the case's transform length,
 // which is uniform over the wavefront
@@ -836,7 +864,7 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2))) void k
   extern __shared__ double2 lds[];
   const uint2 mp = map[blockIdx.x];
   const RowArgs& a = tab[mp.x];
-  switch (31 - __clz(a.m)) {
+  switch (row_form_batch(31 - __clz(a.m))) {
 #define SBFS_DCT2_CASE(LG)                                                                              \
   case LG: {                                                                                            \
     using F = WaveFft<LG>;                                                                              \
@@ -844,7 +872,7 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2))) void k
     dct2_wave<LG, false>(a.rhs, a.buf, a.ny, ((int)mp.y * units + u) * F::R, a.tw, a.t1, a.t2,                   \
                   lds + (size_t)u * F::R * F::PM, (int)threadIdx.x % F::U);                              \
   } break;
-    SBFS_LOG_CASES(SBFS_DCT2_CASE)
+    SBFS_BATCH_CASES(SBFS_DCT2_CASE)
 #undef SBFS_DCT2_CASE
   }
 }
@@ -878,15 +906,15 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2))) void k
   const int K = a.L - 1;
   const ModeSrc src{a.buf, a.X, a.L ? a.ptab + (size_t)2 * K * a.nx : nullptr,
                     a.L ? a.ptab + (size_t)3 * K * a.nx : nullptr, a.nx, a.L, a.P};
-  switch (31 - __clz(a.m)) {
+  switch (row_form_batch(31 - __clz(a.m))) {
 #define SBFS_DCT3_CASE(LG)                                                                              \
   case LG: {                                                                                            \
     using F = WaveFft<LG>;                                                                              \
     const int units = (int)blockDim.x / F::U, u = (int)threadIdx.x / F::U;                              \
-    dct3_wave<LG, true, 0, false>(src, a.ny, ((int)mp.y * units + u) * F::R, a.tw, a.t1, a.t2, a.psi,              \
+    dct3_wave<LG, true, F::SHORT ? 3 : 0, false>(src, a.ny, ((int)mp.y * units + u) * F::R, a.tw, a.t1, a.t2, a.psi,              \
                         lds + (size_t)u * F::R * F::PM, (int)threadIdx.x % F::U);                        \
   } break;
-    SBFS_LOG_CASES(SBFS_DCT3_CASE)
+    SBFS_BATCH_CASES(SBFS_DCT3_CASE)
 #undef SBFS_DCT3_CASE
   }
 }
@@ -997,7 +1025,7 @@ static int poisson_tail(const domain_t* d, PoissonPlan* p, fluid_t* f) {
   double* psi = (double*)f->psi[1].data;
   SBFS_REQUIRE(((uintptr_t)psi & 15) == 0, "poisson: psi[1] must be 16-byte aligned (hipMalloc'ed)");
   const bool nt = stream_fields(nx, ny);
-  switch (ilog2(m)) {
+  switch (row_form(m, ny)) {
 #define SBFS_TAIL_CASE(LG)                                                                          \
   case LG:                                                                                          \
     SBFS_TIMED("k_dct3_psi", hipLaunchKernelGGL((nt ? k_dct3_psi<LG, true> : k_dct3_psi<LG, false>),      \
@@ -1005,7 +1033,7 @@ static int poisson_tail(const domain_t* d, PoissonPlan* p, fluid_t* f) {
                                                 wave_fft_lds(LG), stream(), src, psi, ny, p->tw, p->t1,    \
                                                 p->t2));                                            \
     break;
-    SBFS_LOG_CASES(SBFS_TAIL_CASE)
+    SBFS_FORM_CASES(SBFS_TAIL_CASE)
 #undef SBFS_TAIL_CASE
   }
   return check_launch("poisson: DCT-III + psi");
@@ -1024,7 +1052,7 @@ int poisson_transform_fused(const domain_t* d, DomainCtx* c, fluid_t* f, double*
   }
   const int ny = p->ny;
   const bool nt = stream_fields(p->nx, ny);
-  switch (ilog2(p->m)) {
+  switch (row_form(p->m, ny)) {
 #define SBFS_ROWS_CASE(LG)                                                                              \
   case LG:                                                                                              \
     SBFS_TIMED("k_dct2_rows", hipLaunchKernelGGL((nt ? k_dct2_rows<LG, true> : k_dct2_rows<LG, false>),    \
@@ -1032,7 +1060,7 @@ int poisson_transform_fused(const domain_t* d, DomainCtx* c, fluid_t* f, double*
                                                  wave_fft_lds(LG), stream(), (const double*)p->rhs, p->buf,  \
                                                  ny, p->tw, p->t1, p->t2));                             \
     break;
-    SBFS_LOG_CASES(SBFS_ROWS_CASE)
+    SBFS_FORM_CASES(SBFS_ROWS_CASE)
 #undef SBFS_ROWS_CASE
   }
   if (check_launch("poisson: DCT-II")) return 1;
@@ -1111,7 +1139,7 @@ extern "C" int sbfs_dct_rows(int inverse, size_t n, size_t howmany, const double
   SBFS_HIP(hipMemcpy(dt1, t1.data(), sizeof(double) * t1.size(), hipMemcpyHostToDevice));
   SBFS_HIP(hipMemcpy(dt2, t2.data(), sizeof(double) * t2.size(), hipMemcpyHostToDevice));
   const int rows = (int)howmany;
-  switch (ilog2(m)) {
+  switch (row_form(m, rows)) {
 #define SBFS_TEST_CASE(LG)                                                                                 \
   case LG:                                                                                                 \
     if (inverse)                                                                                           \
@@ -1121,7 +1149,7 @@ extern "C" int sbfs_dct_rows(int inverse, size_t n, size_t howmany, const double
       hipLaunchKernelGGL((k_dct2_rows<LG, false>), dim3(cdiv(rows, WaveFft<LG>::R)), dim3(WaveFft<LG>::U), wave_fft_lds(LG), stream(), \
                          din, dout, rows, dtw, dt1, dt2);                                                  \
     break;
-    SBFS_LOG_CASES(SBFS_TEST_CASE)
+    SBFS_FORM_CASES(SBFS_TEST_CASE)
 #undef SBFS_TEST_CASE
   }
   int rc = check_launch("sbfs_dct_rows");

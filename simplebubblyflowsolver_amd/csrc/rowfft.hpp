@@ -1,4 +1,4 @@
-// Row transforms with one wavefront per group of rows.
+// Row transforms with one wavefront (or a few) per group of rows.
 //
 // The complex FFT is the Stockham autosort sequence of fft_lds (poisson.hip):
 // radix-4 stages with strides s = 1, 4, 16, ... and a final radix-2 stage
@@ -18,6 +18,10 @@
 //    stores them with all 64 lanes;
 //  * M = 2048 takes G = 128 lanes (two wavefronts and a barrier), so every
 //    length keeps 16 points per lane and the same register footprint;
+//  * the short form has 4 points per lane and one radix-4 stage per pass, with
+//    the twiddles of all passes loaded before the row: four times the
+//    lanes and a quarter of the work of each, for grids whose rows leave the chip
+//    idle (64 x 128 takes 16 wavefronts instead of 4);
 //  * the buffer is padded by one point in 16 so that the stride-16 stores
 //    of the first pass spread over the LDS banks.
 // A "unit" is the U = R G threads that share one group of rows.
@@ -39,17 +43,25 @@ __device__ __forceinline__ double2 wmul(double2 a, double2 b) {
   return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
 }
 
-__host__ __device__ constexpr int wave_fft_g(int log) { return log >= 4 ? (1 << log) / 16 : 1; }
-__host__ __device__ constexpr int wave_fft_r(int log) { return wave_fft_g(log) >= 64 ? 1 : 64 / wave_fft_g(log); }
-__host__ __device__ constexpr int wave_fft_u(int log) { return wave_fft_r(log) * wave_fft_g(log); }
+// A form is log2(M), or that plus kShort: 4 points per lane.
+constexpr int kShort = 16;
+__host__ __device__ constexpr int wave_fft_g(int form) {
+  const int log = form & (kShort - 1);
+  return form >= kShort ? (1 << log) / 4 : log >= 4 ? (1 << log) / 16 : 1;
+}
+__host__ __device__ constexpr int wave_fft_r(int form) { return wave_fft_g(form) >= 64 ? 1 : 64 / wave_fft_g(form); }
+__host__ __device__ constexpr int wave_fft_u(int form) { return wave_fft_r(form) * wave_fft_g(form); }
 
-template <int LOG>
+template <int FORM>
 struct WaveFft {
+  static constexpr int LOG = FORM & (kShort - 1);
+  static constexpr bool SHORT = FORM >= kShort;
+  static_assert(!SHORT || LOG >= 2, "4 points per lane");
   static constexpr int M = 1 << LOG;           // complex points
   static constexpr int N = 2 * M;              // real points
-  static constexpr int G = wave_fft_g(LOG);    // lanes per row
-  static constexpr int R = wave_fft_r(LOG);    // rows per unit
-  static constexpr int U = wave_fft_u(LOG);    // threads per unit: 64, or 128 for M = 2048
+  static constexpr int G = wave_fft_g(FORM);   // lanes per row
+  static constexpr int R = wave_fft_r(FORM);   // rows per unit
+  static constexpr int U = wave_fft_u(FORM);   // threads per unit: 64, or G where that is more
   static constexpr int PM = M + (M >> 4);      // padded buffer, points
   static constexpr int NR4 = LOG / 2;          // radix-4 stages
   static __device__ __forceinline__ void sync() {
@@ -59,8 +71,9 @@ struct WaveFft {
 };
 
 // LDS bytes of one unit's rows
-__host__ __device__ constexpr size_t wave_fft_lds(int log) {
-  return sizeof(double2) * (size_t)wave_fft_r(log) * (size_t)((1 << log) + ((1 << log) >> 4));
+__host__ __device__ constexpr size_t wave_fft_lds(int form) {
+  const int m = 1 << (form & (kShort - 1));
+  return sizeof(double2) * (size_t)wave_fft_r(form) * (size_t)(m + (m >> 4));
 }
 
 // radix-4 butterfly of fft_lds: outputs 1..3 take the twiddles w1..w3
@@ -91,11 +104,31 @@ struct TwSet {
   double2 w[N];
 };
 
-template <int LOG, int T>
+// (the short form's passes are over before the next one's twiddles arrive: all
+// of its sets are loaded before the row, 3 twiddles each)
+template <int NR4>
+struct TwShort {
+  TwSet<3> r4[NR4];
+  TwSet<1> r2;
+};
+
+template <int FORM, int T>
 __device__ __forceinline__ auto pass_tw(int lt, const double2* __restrict__ tw) {
-  using F = WaveFft<LOG>;
+  using F = WaveFft<FORM>;
   constexpr int M = F::M, NR4 = F::NR4;
-  if constexpr (T + 1 < NR4) {  // stages T, T+1 (one group of 4 + 4 butterflies per lane)
+  if constexpr (F::SHORT) {
+    static_assert(T == 0, "all sets at once");
+    TwShort<NR4> t;
+#pragma unroll
+    for (int k = 0; k < NR4; k++) {
+      const int ps = (lt >> (2 * k)) << (2 * k);
+      t.r4[k].w[0] = tw[ps];
+      t.r4[k].w[1] = tw[2 * ps];
+      t.r4[k].w[2] = tw[3 * ps];
+    }
+    t.r2.w[0] = tw[0];
+    return t;
+  } else if constexpr (T + 1 < NR4) {  // stages T, T+1 (one group of 4 + 4 butterflies per lane)
     static_assert((M / 16) / F::G == 1, "one group per lane");
     constexpr int s = 1 << (2 * T), Q = M / (16 * s);
     TwSet<15> t;
@@ -122,7 +155,7 @@ __device__ __forceinline__ auto pass_tw(int lt, const double2* __restrict__ tw) 
       t.w[3 * i + 2] = tw[3 * p * s];
     }
     return t;
-  } else if constexpr (LOG & 1) {  // the final radix-2 stage
+  } else if constexpr (F::LOG & 1) {  // the final radix-2 stage
     TwSet<1> t;
     t.w[0] = tw[0];
     return t;
@@ -134,9 +167,9 @@ __device__ __forceinline__ auto pass_tw(int lt, const double2* __restrict__ tw) 
 // stages T and T+1 (s = 4^T): group (p2, q) runs the stage-T butterflies
 // p = p2 + k2 Q (k2 = 0..3) at q, whose outputs k are the inputs of the
 // stage-(T+1) butterfly (p2, q + s k)
-template <int LOG, int T, typename Ld>
+template <int FORM, int T, typename Ld>
 __device__ __forceinline__ void pass_pair(double2* Z, int lt, const TwSet<15>& t, Ld ld) {
-  using F = WaveFft<LOG>;
+  using F = WaveFft<FORM>;
   constexpr int M = F::M, s = 1 << (2 * T), q4 = M / (4 * s), Q = q4 / 4;
   const int q = lt & (s - 1), p2 = lt >> (2 * T);
   double2 r[16];
@@ -162,9 +195,9 @@ __device__ __forceinline__ void pass_pair(double2* Z, int lt, const TwSet<15>& t
 }
 
 // one radix-4 stage T (the last one when their count is odd)
-template <int LOG, int T, typename Ld, int N>
+template <int FORM, int T, typename Ld, int N>
 __device__ __forceinline__ void pass_r4(double2* Z, int lt, const TwSet<N>& t, Ld ld) {
-  using F = WaveFft<LOG>;
+  using F = WaveFft<FORM>;
   constexpr int M = F::M, s = 1 << (2 * T), q4 = M / (4 * s);
   constexpr int PER = (M / 4) / F::G;
   static_assert(N == 3 * PER, "twiddles of the stage");
@@ -188,9 +221,9 @@ __device__ __forceinline__ void pass_r4(double2* Z, int lt, const TwSet<N>& t, L
 }
 
 // the final radix-2 stage (s = M / 2)
-template <int LOG, typename Ld>
+template <int FORM, typename Ld>
 __device__ __forceinline__ void pass_r2(double2* Z, int lt, const TwSet<1>& t, Ld ld) {
-  using F = WaveFft<LOG>;
+  using F = WaveFft<FORM>;
   constexpr int s = F::M / 2;
   constexpr int PER = s / F::G;
   double2 r0[PER], r1[PER];
@@ -212,35 +245,50 @@ __device__ __forceinline__ void pass_r2(double2* Z, int lt, const TwSet<1>& t, L
   F::sync();
 }
 
+// the short form's stages from T on
+template <int FORM, int T, typename Ld, typename Tw>
+__device__ __forceinline__ void fft_short(double2* Z, int lt, Ld ld, const Tw& t) {
+  using F = WaveFft<FORM>;
+  if constexpr (T < F::NR4) {
+    pass_r4<FORM, T>(Z, lt, t.r4[T], ld);
+    fft_short<FORM, T + 1>(Z, lt, ZLoad{Z}, t);
+  } else if constexpr (F::LOG & 1) {
+    pass_r2<FORM>(Z, lt, t.r2, ld);
+  }
+}
+
 // the stages from T on, with the twiddles of the pass at T already loaded;
 // the first pass reads its input through `ld`
-template <int LOG, int T, typename Ld, typename Tw>
+template <int FORM, int T, typename Ld, typename Tw>
 __device__ __forceinline__ void fft_from(double2* Z, int lt, const double2* __restrict__ tw, Ld ld, const Tw& cur) {
-  constexpr int NR4 = WaveFft<LOG>::NR4;
+  using F = WaveFft<FORM>;
+  constexpr int NR4 = F::NR4;
   if constexpr (T + 1 < NR4) {
-    const auto nxt = pass_tw<LOG, T + 2>(lt, tw);
-    pass_pair<LOG, T>(Z, lt, cur, ld);
-    fft_from<LOG, T + 2>(Z, lt, tw, ZLoad{Z}, nxt);
+    const auto nxt = pass_tw<FORM, T + 2>(lt, tw);
+    pass_pair<FORM, T>(Z, lt, cur, ld);
+    fft_from<FORM, T + 2>(Z, lt, tw, ZLoad{Z}, nxt);
   } else if constexpr (T < NR4) {
-    const auto nxt = pass_tw<LOG, T + 1>(lt, tw);
-    pass_r4<LOG, T>(Z, lt, cur, ld);
-    fft_from<LOG, T + 1>(Z, lt, tw, ZLoad{Z}, nxt);
-  } else if constexpr (LOG & 1) {
-    pass_r2<LOG>(Z, lt, cur, ld);
+    const auto nxt = pass_tw<FORM, T + 1>(lt, tw);
+    pass_r4<FORM, T>(Z, lt, cur, ld);
+    fft_from<FORM, T + 1>(Z, lt, tw, ZLoad{Z}, nxt);
+  } else if constexpr (F::LOG & 1) {
+    pass_r2<FORM>(Z, lt, cur, ld);
   }
 }
 
 // forward M-point FFT of the points ld(0..M-1) into Z (natural order);
-// tw0 = pass_tw<LOG, 0>(lt, tw), loaded by the caller as early as it likes
-template <int LOG, typename Ld, typename Tw>
+// tw0 = pass_tw<FORM, 0>(lt, tw), loaded by the caller as early as it likes
+template <int FORM, typename Ld, typename Tw>
 __device__ __forceinline__ void wave_fft(double2* Z, int lt, const double2* __restrict__ tw, Ld ld, const Tw& tw0) {
-  if constexpr (LOG == 0) {
+  if constexpr (WaveFft<FORM>::LOG == 0) {
     const double2 v = ld(0);
     wave_sync();
     Z[0] = v;
     wave_sync();
+  } else if constexpr (WaveFft<FORM>::SHORT) {
+    fft_short<FORM, 0>(Z, lt, ld, tw0);
   } else {
-    fft_from<LOG, 0>(Z, lt, tw, ld, tw0);
+    fft_from<FORM, 0>(Z, lt, tw, ld, tw0);
   }
 }
 
