@@ -217,6 +217,7 @@ __device__ __forceinline__ void tile_body(const MarchArgs& a, int bx, int by) {
   put_r(S_GX, g0x);
   put_r(S_GY, g0y);
   __syncthreads();
+  if (s > je + 2) return;
   if (CORR) {
     uxm = get_d(S_UX, wm);
     uxp = get_d(S_UX, wp);
@@ -270,6 +271,7 @@ __device__ __forceinline__ void tile_body(const MarchArgs& a, int bx, int by) {
   put_r(S_K, k0);
   put_r(S_MFX, mfx0);
   __syncthreads();
+  if (s < jb - 1) return;
   // -- 3: fluxes through the bottom face of row s, stresses -------------------
   R fy0 = 0, mfy0 = 0;
   {
@@ -315,6 +317,7 @@ __device__ __forceinline__ void tile_body(const MarchArgs& a, int bx, int by) {
   put_r(S_TXY, txy0);
   put_r(S_CTYY, cyc_tyy0);
   __syncthreads();
+  if (s > je + 1) return;
   // -- 4: new vof (update/main.c:54-120) and density, momentum fluxes ----------
   const R fyp1 = get_r(S_FY, wp), mfyp1 = get_r(S_MFY, wp), txy1 = get_r(S_TXY, wp);
   const R mfym1 = get_r(S_MFY, wm), mfxm1 = get_r(S_MFX, wm), cyc_tyym1 = get_r(S_CTYY, wm);
@@ -345,6 +348,7 @@ __device__ __forceinline__ void tile_body(const MarchArgs& a, int bx, int by) {
   const R qy_uy_new = (SB(T_ECY) * mfy0 + SB(T_ECY) * mfyp1) * (R(0.5) * ruy0 + R(0.5) * ruyp1);
   const R cyf_txy0 = SB(T_CYF) * txy0, cyf_txy1 = SB(T_CYF) * txy1;
   __syncthreads();
+  if (s < jb) return;
   // -- 5: predicted velocity (predict/ux.c, uy.c, force.c), outputs ------------
   const double dnm1 = get_d(S_DN, wm);
   const R km1 = get_r(S_K, wm);
