@@ -505,6 +505,9 @@ static int tile_rows(int nx, int ny, bool mixed) {
 // its bands are short (48 rows on the 2048 x 4096 swarm), two when one round
 // would give bands of 160 rows or more (4096 x 8192: 96-row bands, 6.16 ms
 // per mixed step against 6.22 with 191 rows; 128 rows 6.32, ordered 6.47-7.0).
+// Where a round has room for shorter bands, the ring fill costs more than the
+// idle slots: 5 rows at least in mixed precision (512 x 1024, three stages: 4 rows
+// 108 us, 5 rows 104, 6 rows 112).
 // SBFS_MARCH_BAND overrides the choice.
 static int march_band(int nx, int ny, bool mixed) {
   static long slots[2] = {0, 0};
@@ -533,7 +536,8 @@ static int march_band(int nx, int ny, bool mixed) {
     bands = quarters * slots_now / (4 * strips);
   }
   long band = (ny + bands - 1) / bands;
-  if (band < 4) band = 4;
+  const long least = mixed ? 5 : 4;
+  if (band < least) band = least;
   return (int)(band < ny ? band : ny);
 }
 

@@ -38,9 +38,16 @@ namespace sbfs {
 // only what it wrote, so no barrier is needed).  The FP64 body has: with them
 // in LDS its folded kernel took 355 us instead of 352 at 2048 x 4096.
 enum { RG_QUXS, RG_CYCUYS, RG_D1X, RG_CGY, RG_PSM1, RG_PM1, RG_DNM1, RG_N };
-template <bool LR>
+// The FP32 body's FP64 tables are the four that its FP64 parts read (fp64_slot).
+template <typename R>
+constexpr int fp64_slot(int t) {
+  return std::is_same<R, double>::value ? t : t == T_RHF ? 0 : t == T_RJC ? 1 : t == T_QF ? 2 : t == T_CYC ? 3 : -1;
+}
+template <typename R, bool LR>
 struct MarchLds {
-  double st[T_N][64];
+  static constexpr bool kSingle = std::is_same<R, float>::value;
+  double st[kSingle ? 4 : T_N][64];
+  float sf[kSingle ? T_N : 1][64];
   double rings[LR ? RG_N : 1][64];
 };
 template <typename R, bool CORR>
@@ -57,7 +64,7 @@ constexpr bool kLdsRings = CORR && std::is_same<R, float>::value;
 // NT: the FP64 bodies store their output rows streaming (see ST below)
 template <typename R, bool CORR, bool NT, bool IN>
 __device__ __forceinline__ void march_body(const MarchArgs& a, int bx, int by,
-                                           MarchLds<kLdsRings<R, CORR>>& lds) {
+                                           MarchLds<R, kLdsRings<R, CORR>>& lds) {
   using A = Arith<R>;
   using V3 = V3R<R>;
   auto& st = lds.st;
@@ -81,51 +88,49 @@ __device__ __forceinline__ void march_body(const MarchArgs& a, int bx, int by,
   const bool c_first = !IN && c == 1, c_last = !IN && c == nx;
   const bool c_out = c >= i0 && c < i0 + kStrip && (IN || c <= nx);
   const int cc = c < 0 ? 0 : (c > nx + 1 ? nx + 1 : c);
+  // The column tables and dt are loaded first and used last before the row
+  // loop, after the first rows' loads have been issued: the wavefront waits for
+  // memory once, not for each in turn, which was 6 of 31 us at 512 x 1024
+  // mixed (k_march at 1024 x 2048 103 -> 98 us, with the fold 127 -> 119).
+  double tab[T_N];
   {
     const double* tabs[T_N] = {a.cf.rhf, a.cf.rhc, a.cf.rjf, a.cf.rjc, a.cf.qf, a.cf.qc, a.cf.eqf,
                                a.cf.ecy, a.cf.cyc, a.cf.cyf, a.cf.dfx, a.cf.dcx, a.hxxf1, a.hxxc1};
 #pragma unroll
-    for (int t = 0; t < T_N; t++) st[t][lane] = tabs[t][cc];
+    for (int t = 0; t < T_N; t++) tab[t] = tabs[t][cc];
   }
+  const double dt_in = *a.dt;
   constexpr bool LR = kLdsRings<R, CORR>;
-  if (LR)
-    for (int k = 0; k < RG_N; k++) rings[k][lane] = 0.;
-  __syncthreads();
   const int ll = lane > 0 ? lane - 1 : 0, lr = lane < 63 ? lane + 1 : 63;
   // tables in FP64 (the FP64 parts) and in the stencil type
-  auto TB = [&](int t) { return st[t][lane]; };
-  auto TR = [&](int t) { return st[t][lr]; };
-  auto SB = [&](int t) { return R(st[t][lane]); };
-  auto SL = [&](int t) { return R(st[t][ll]); };
-  auto SR = [&](int t) { return R(st[t][lr]); };
+  // (those in FP32 are rounded once here: converted at each use they cost 20
+  // instructions per row step, k_march_mixed 194 -> 188 us at 2048 x 4096)
+  auto TB = [&](int t) { return st[fp64_slot<R>(t)][lane]; };
+  auto TR = [&](int t) { return st[fp64_slot<R>(t)][lr]; };
+  auto stencil = [&](int t, int l) {
+    if constexpr (std::is_same<R, float>::value) return lds.sf[t][l];
+    else return st[t][l];
+  };
+  auto SB = [&](int t) { return stencil(t, lane); };
+  auto SL = [&](int t) { return stencil(t, ll); };
+  auto SR = [&](int t) { return stencil(t, lr); };
   // x / HXXF of the lane's column and x / hy: divided in the FP64 body,
   // multiplied by the stored reciprocals in the mixed one
   constexpr bool kExactQ = std::is_same<R, double>::value;
-  auto per_h = [&](double x) { return kExactQ ? x / TB(T_HXXF) : x * TB(T_RHF); };
+  auto per_h = [&](double x) {
+    if constexpr (kExactQ) return x / TB(T_HXXF);
+    else return x * TB(T_RHF);
+  };
   const double hy = a.hy, rhy = a.cf.rhy;
   auto per_hy = [&](double x) { return kExactQ ? x / hy : x * rhy; };
   const R hyr = uni(R(hy)), rhyr = uni(R(rhy));
-  const double dt = uni(*a.dt);
-  // (dt * a.ca equals a.ca * dt bit for bit)
-  const double dtca = uni(dt * a.ca), dtcb = uni(dt * a.cb), dtcg = uni(dt * a.cg);
-  const double dt_old = a.g_old * dt, dt_new = a.g_new * dt;
-  const double c0 = uni(1. / a.norm / dt_new * a.refden);
-  const double c1 = uni(1. / a.norm * -1. / dt_new * dt_old);
   const bool has_b = a.stage != 0;
-  const R denr1 = uni(R(a.denr) - R(1));
-  // the previous stage's projection (correct_velocity/ux.c, uy.c): the same
-  // expressions as k_post, with the lane's face distance in the divisions
-  const double pdtn = a.pg_new * dt, pdto = a.pg_old * dt;
-  const double pcoef = -1. / pdtn * pdto;
-  const double pdtc = uni(pdtn * pcoef), irefden = uni(1. / a.refden);
-  const R refdeninv = uni(R(a.refdeninv)), tension = uni(R(a.tension)), grav = uni(R(a.grav));
 
-  // Rows of each layout, shifted to lane 0's column: a pinned row pointer
-  // (FP32 bodies) or a (field, byte offset) pair (FP64 bodies), see RowRef.
+  // Rows of each layout, shifted to lane 0's column: a (field, byte offset)
+  // pair, see RowRef.
   const ptrdiff_t wc = nx + 2, wf = nx + 1;
   auto row = [&](auto* f, ptrdiff_t e) {
-    if constexpr (std::is_same<R, float>::value) return f + e;
-    else return RowRef<std::remove_reference_t<decltype(*f)>>{f, (unsigned)(e * (ptrdiff_t)sizeof(*f))};
+    return RowRef<std::remove_reference_t<decltype(*f)>>{f, (unsigned)(e * (ptrdiff_t)sizeof(*f))};
   };
   auto vof_row = [&](auto* f, int j) { return row(f, (ptrdiff_t)(j + 1) * wc + cl); };         // L::vof
   auto cc_row = [&](auto* f, int j) { return row(f, (ptrdiff_t)j * wc + cl); };                // L::cc
@@ -184,7 +189,6 @@ __device__ __forceinline__ void march_body(const MarchArgs& a, int bx, int by,
   double q_uxs_m1 = 0., cyc_uys_m1 = 0.;                    // rhs terms of row s-1
   double d1x_m1 = 0., d1y = 0., cg_ym = 0.;                 // rhs densities / y gradient
   const int s_first = jb - (CORR ? kWarmCorr : kWarm);
-  const double pcx0 = uni(pdtn / a.refden), pcy = uni(pdtn / a.refden / hy);
   auto ring_ld = [&](int k, double reg) { return LR ? rings[k][lane] : reg; };
   auto ring_st = [&](int k, double& reg, double v) {
     if (LR) rings[k][lane] = v;
@@ -254,6 +258,28 @@ __device__ __forceinline__ void march_body(const MarchArgs& a, int bx, int by,
   // so the first step's corner gradients are already valid
   vp1 = ld_vof(wrap_r(s_first, ny));
   vp2 = ld_vof(w1);
+#pragma unroll
+  for (int t = 0; t < T_N; t++) {
+    if (fp64_slot<R>(t) >= 0) st[fp64_slot<R>(t)][lane] = tab[t];
+    if (lds.kSingle) lds.sf[t][lane] = float(tab[t]);
+  }
+  if (LR)
+    for (int k = 0; k < RG_N; k++) rings[k][lane] = 0.;
+  __syncthreads();
+  const double dt = uni(dt_in);
+  // (dt * a.ca equals a.ca * dt bit for bit)
+  const double dtca = uni(dt * a.ca), dtcb = uni(dt * a.cb), dtcg = uni(dt * a.cg);
+  const double dt_old = a.g_old * dt, dt_new = a.g_new * dt;
+  const double c0 = uni(1. / a.norm / dt_new * a.refden);
+  const double c1 = uni(1. / a.norm * -1. / dt_new * dt_old);
+  const R denr1 = uni(R(a.denr) - R(1));
+  // the previous stage's projection (correct_velocity/ux.c, uy.c): the same
+  // expressions as k_post, with the lane's face distance in the divisions
+  const double pdtn = a.pg_new * dt, pdto = a.pg_old * dt;
+  const double pcoef = -1. / pdtn * pdto;
+  const double pdtc = uni(pdtn * pcoef), irefden = uni(1. / a.refden);
+  const R refdeninv = uni(R(a.refdeninv)), tension = uni(R(a.tension)), grav = uni(R(a.grav));
+  const double pcx0 = uni(pdtn / a.refden), pcy = uni(pdtn / a.refden / hy);
   asm volatile("" : "+v"(vp1), "+v"(vp2));
   fence();
   unsigned weight = 0;  // marched rows with an interface cell
@@ -763,7 +789,7 @@ __device__ __forceinline__ bool march_unit(const MarchArgs& a, int& bx, int& by)
 __device__ __forceinline__ bool march_inner(int nx, int bx) { return bx >= 1 && 1 + bx * kStrip + 60 <= nx; }
 template <typename R, bool CORR, bool NT>
 __device__ __forceinline__ void march_strip(const MarchArgs& a, int bx, int by) {
-  __shared__ MarchLds<kLdsRings<R, CORR>> lds;
+  __shared__ MarchLds<R, kLdsRings<R, CORR>> lds;
   if (std::is_same<R, double>::value && march_inner(a.nx, bx)) march_body<R, CORR, NT, true>(a, bx, by, lds);
   else march_body<R, CORR, NT, false>(a, bx, by, lds);
 }

@@ -38,16 +38,16 @@ __device__ __forceinline__ double from_right(double v) {
 // base plus the lane's byte offset:
 //  * lane_at: the row's 64-bit address, pinned to SGPRs (readfirstlane of a
 //    uniform value), plus the lane offset; all arrays share one offset VGPR.
-//    The FP32 bodies use it: they run three wavefronts per SIMD at 168 VGPRs
-//    and have none to spare.
+//    The tile kernel uses it, which addresses every row once.
 //  * RowRef: the field's base and a 32-bit byte offset of lane 0's element,
 //    plus the lane offset; rows of one layout share one offset for all
 //    their fields, where a 64-bit row address per field and row costs
-//    several scalar or vector operations.  The FP64 bodies use it (2 %
-//    faster there; in the FP32 bodies its offsets push the register count
-//    into scratch).  The fused path keeps every field below 4 GiB.  Lanes
-//    whose column lies before the array wrap the 32-bit offset; they are
-//    the masked halo lanes and access nothing.
+//    several scalar operations.  The marching kernels use it: a row step of the
+//    mixed body has 372 scalar instructions with it instead of 777, and a
+//    wavefront issues one instruction at a time (k_march_mixed 55.5 -> 50 us
+//    at 1024 x 1500, together with the tables in FP32).  The fused path keeps
+//    every field below 4 GiB.  Lanes whose column lies before the array wrap
+//    the 32-bit offset; they are the masked halo lanes and access nothing.
 // Both go through a global-address-space pointer, so the accesses stay
 // global_load / global_store (a generic pointer made from an integer would
 // compile to flat accesses, which also count against the LDS wait counter).
