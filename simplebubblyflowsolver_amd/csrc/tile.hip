@@ -96,7 +96,9 @@ __device__ __forceinline__ void tile_body(const MarchArgs& a, int bx, int by) {
     return mixr<R>(a.visr, a.vlo, a.vhi, v);
   };
   auto VISUY = [&](R vb, R vt) { return mixr<R>(a.visr, a.vlo, a.vhi, R(0.5) * vb + R(0.5) * vt); };
-  auto rw = [&](auto* f, ptrdiff_t e) { return f + e; };
+  auto rw = [&](auto* f, ptrdiff_t e) {
+    return RowRef<std::remove_reference_t<decltype(*f)>>{f, (unsigned)(e * (ptrdiff_t)sizeof(*f))};
+  };
   const ptrdiff_t wc = nx + 2, wf = nx + 1;
   auto vof_row = [&](auto* f, int j) { return rw(f, (ptrdiff_t)(j + 1) * wc + cl); };         // L::vof
   auto cc_row = [&](auto* f, int j) { return rw(f, (ptrdiff_t)j * wc + cl); };                // L::cc
