@@ -440,6 +440,8 @@ __global__ void k_march_nt(const MarchArgs* a);          // k_march with streami
 __global__ void k_march_corr_nt(const MarchArgs* a);     // k_march_corr with streaming output stores
 __global__ void k_march_mixed(const MarchArgs* a);       // FP32 stencils
 __global__ void k_march_mixed_corr(const MarchArgs* a);  // FP32 stencils + projection
+__global__ void k_march_mixed_wide(const MarchArgs* a);       // k_march_mixed, fields of 4 GiB or more
+__global__ void k_march_mixed_corr_wide(const MarchArgs* a);  // k_march_mixed_corr, fields of 4 GiB or more
 
 // Stages 1 and 2 fold the previous stage's projection and pressure update
 // into their stage kernel (k_march_corr), which reads the predicted velocity,
@@ -483,6 +485,7 @@ int tile_rows(unsigned short_groups, unsigned tall_groups, bool mixed) {
   return tall_groups <= (mixed ? 640u : 1024u) ? kTileTall : 0;
 }
 static int tile_rows(int nx, int ny, bool mixed) {
+  if (!fp64_march_addressable(nx, ny) || (mixed && mixed_march_wide(nx, ny))) return 0;
   return tile_rows(tile_groups(nx, ny, kTileShort), tile_groups(nx, ny, kTileTall), mixed);
 }
 
@@ -721,6 +724,7 @@ static int fused_body(const domain_t* domain, DomainCtx* c, fluid_t* fluid, inte
   // them (the previous step's; the bubbles move a fraction of a cell per
   // step), for all three stages of this step
   const bool mixed = options().precision == SBFS_PRECISION_MIXED;
+  const bool wide = mixed && mixed_march_wide(nx, ny);
   const int tile = tile_rows(nx, ny, mixed);
   const bool ordered = tile == 0 && march_ordered(mixed);
   const int units = march_units(nx, ny, band);
@@ -766,9 +770,9 @@ static int fused_body(const domain_t* domain, DomainCtx* c, fluid_t* fluid, inte
       if (tile) {
         tile_launch(ma, nx, ny, tile, mixed, corr);
       } else if (mixed && corr)
-        SBFS_TIMED("k_march_mixed_corr", hipLaunchKernelGGL(k_march_mixed_corr, grid, block, 0, stream(), ma));
+        SBFS_TIMED("k_march_mixed_corr", hipLaunchKernelGGL((wide ? k_march_mixed_corr_wide : k_march_mixed_corr), grid, block, 0, stream(), ma));
       else if (mixed)
-        SBFS_TIMED("k_march_mixed", hipLaunchKernelGGL(k_march_mixed, grid, block, 0, stream(), ma));
+        SBFS_TIMED("k_march_mixed", hipLaunchKernelGGL((wide ? k_march_mixed_wide : k_march_mixed), grid, block, 0, stream(), ma));
       else if (corr)
         SBFS_TIMED("k_march_corr", hipLaunchKernelGGL((nt ? k_march_corr_nt : k_march_corr), grid, block, 0, stream(), ma));
       else
@@ -866,7 +870,7 @@ static StepKey step_key(const DomainCtx* c, fluid_t* f, interface_t* s, const Co
   key_add(k, scr.cut);
   const bool mixed = options().precision == SBFS_PRECISION_MIXED;
   k.v.push_back((march_ordered(mixed) ? 1 : 0) | ((uint64_t)tile_rows((int)c->nx, (int)c->ny, mixed) << 1));
-  k.v.push_back(stream_fields(c->nx, c->ny) ? 1 : 0);
+  k.v.push_back((stream_fields(c->nx, c->ny) ? 1 : 0) | (mixed_march_wide(c->nx, c->ny) ? 2 : 0));
   key_add(k, scr.order);
   k.v.push_back(c->epoch);
   k.v.push_back(poisson_epoch(c));

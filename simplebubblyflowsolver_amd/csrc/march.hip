@@ -61,12 +61,14 @@ constexpr bool kLdsRings = CORR && std::is_same<R, float>::value;
 // (bx, by): the strip and band of this wavefront
 // IN: every lane of the strip holds an interior cell that touches no wall
 // (march_inner): only the interface and the strip's output columns mask lanes
-// NT: the FP64 bodies store their output rows streaming (see ST below)
-template <typename R, bool CORR, bool NT, bool IN>
+// ALT: the FP64 bodies store their output rows streaming (see ST below); the
+// FP32 ones address rows by 64 bits (see row below)
+template <typename R, bool CORR, bool ALT, bool IN>
 __device__ __forceinline__ void march_body(const MarchArgs& a, int bx, int by,
                                            MarchLds<R, kLdsRings<R, CORR>>& lds) {
   using A = Arith<R>;
   using V3 = V3R<R>;
+  constexpr bool NT = ALT && std::is_same<R, double>::value, WIDE = ALT && std::is_same<R, float>::value;
   auto& st = lds.st;
   auto& rings = lds.rings;
   const int lane = threadIdx.x;
@@ -127,10 +129,11 @@ __device__ __forceinline__ void march_body(const MarchArgs& a, int bx, int by,
   const bool has_b = a.stage != 0;
 
   // Rows of each layout, shifted to lane 0's column: a (field, byte offset)
-  // pair, see RowRef.
+  // pair, see RowRef, or a row pointer for fields of 4 GiB or more.
   const ptrdiff_t wc = nx + 2, wf = nx + 1;
   auto row = [&](auto* f, ptrdiff_t e) {
-    return RowRef<std::remove_reference_t<decltype(*f)>>{f, (unsigned)(e * (ptrdiff_t)sizeof(*f))};
+    if constexpr (WIDE) return f + e;
+    else return RowRef<std::remove_reference_t<decltype(*f)>>{f, (unsigned)(e * (ptrdiff_t)sizeof(*f))};
   };
   auto vof_row = [&](auto* f, int j) { return row(f, (ptrdiff_t)(j + 1) * wc + cl); };         // L::vof
   auto cc_row = [&](auto* f, int j) { return row(f, (ptrdiff_t)j * wc + cl); };                // L::cc
@@ -144,7 +147,6 @@ __device__ __forceinline__ void march_body(const MarchArgs& a, int bx, int by,
   // measured k_march 1198 -> 1164 us and k_march_corr 1502 -> 1446 us at
   // 4096 x 8192; the FP32 bodies slowed by 4-5 % with it and keep ordinary
   // stores.
-  static_assert(!NT || std::is_same<R, double>::value, "streaming stores in the FP64 bodies only");
   auto ST = [&](auto r, double v) {
     if constexpr (NT) __builtin_nontemporal_store(v, lane_gp(r, loff));
     else AT(r) = v;
@@ -787,11 +789,11 @@ __device__ __forceinline__ bool march_unit(const MarchArgs& a, int& bx, int& by)
 // compute, got slower (2048 x 4096: 206 us against 198, with the fold 273 against 261)
 // and keep the one masked body.
 __device__ __forceinline__ bool march_inner(int nx, int bx) { return bx >= 1 && 1 + bx * kStrip + 60 <= nx; }
-template <typename R, bool CORR, bool NT>
+template <typename R, bool CORR, bool ALT>
 __device__ __forceinline__ void march_strip(const MarchArgs& a, int bx, int by) {
   __shared__ MarchLds<R, kLdsRings<R, CORR>> lds;
-  if (std::is_same<R, double>::value && march_inner(a.nx, bx)) march_body<R, CORR, NT, true>(a, bx, by, lds);
-  else march_body<R, CORR, NT, false>(a, bx, by, lds);
+  if (std::is_same<R, double>::value && march_inner(a.nx, bx)) march_body<R, CORR, ALT, true>(a, bx, by, lds);
+  else march_body<R, CORR, ALT, false>(a, bx, by, lds);
 }
 #define SBFS_MARCH_KERNEL(name, R, CORR, WAVES)                                            \
   __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WAVES))) void name( \
@@ -813,16 +815,19 @@ SBFS_MARCH_KERNEL(k_march_mixed, float, false, SBFS_MIXED_WAVES)
 SBFS_MARCH_KERNEL(k_march_mixed_corr, float, true, SBFS_MIXED_WAVES)
 #undef SBFS_MARCH_KERNEL
 // the FP64 stage kernels with streaming output stores (single cases whose
-// fields the Infinity Cache cannot keep, stream_fields)
-#define SBFS_MARCH_NT_KERNEL(name, CORR)                                                         \
-  __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(SBFS_FP64_WAVES))) void name( \
-      const MarchArgs* __restrict__ args) {                                                      \
-    const MarchArgs& a = *args;                                                                  \
-    int bx, by;                                                                                  \
-    if (march_unit(a, bx, by)) march_strip<double, CORR, true>(a, bx, by);                       \
+// fields the Infinity Cache cannot keep, stream_fields), and the FP32 ones for
+// fields of 4 GiB or more
+#define SBFS_MARCH_ALT_KERNEL(name, R, CORR, WAVES)                                       \
+  __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WAVES))) void name( \
+      const MarchArgs* __restrict__ args) {                                               \
+    const MarchArgs& a = *args;                                                           \
+    int bx, by;                                                                           \
+    if (march_unit(a, bx, by)) march_strip<R, CORR, true>(a, bx, by);                     \
   }
-SBFS_MARCH_NT_KERNEL(k_march_nt, false)
-SBFS_MARCH_NT_KERNEL(k_march_corr_nt, true)
-#undef SBFS_MARCH_NT_KERNEL
+SBFS_MARCH_ALT_KERNEL(k_march_nt, double, false, SBFS_FP64_WAVES)
+SBFS_MARCH_ALT_KERNEL(k_march_corr_nt, double, true, SBFS_FP64_WAVES)
+SBFS_MARCH_ALT_KERNEL(k_march_mixed_wide, float, false, SBFS_MIXED_WAVES)
+SBFS_MARCH_ALT_KERNEL(k_march_mixed_corr_wide, float, true, SBFS_MIXED_WAVES)
+#undef SBFS_MARCH_ALT_KERNEL
 
 }  // namespace sbfs

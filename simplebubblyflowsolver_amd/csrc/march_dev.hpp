@@ -34,22 +34,35 @@ __device__ __forceinline__ double from_right(double v) {
   return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
 }
 
-// A wave-uniform row, so that every access is a scalar base plus a 32-bit byte
-// offset: the field's base, the offset of lane 0's element, and the lane's.  Rows
-// of one layout share one offset for all their fields, where a 64-bit row address
-// per field and row costs several scalar operations: a row step of the mixed
-// marching body has 372 scalar instructions with it instead of 777, and a
-// wavefront issues one instruction at a time (k_march_mixed 55.5 -> 50 us at
-// 1024 x 1500, together with the tables in FP32; k_tile 27.9 -> 27.4 at
-// 512 x 512).  The fused path keeps every field below 4 GiB.  Lanes whose column
-// lies before the array wrap the 32-bit offset; they are the masked halo lanes and
-// access nothing.
-// It goes through a global-address-space pointer, so the accesses stay
+// Two ways to address a wave-uniform row, so that every access is a scalar
+// base plus the lane's byte offset:
+//  * RowRef: the field's base and a 32-bit byte offset of lane 0's element,
+//    plus the lane offset; rows of one layout share one offset for all
+//    their fields, where a 64-bit row address per field and row costs
+//    several scalar operations: a row step of the mixed marching body has 372
+//    scalar instructions with it instead of 777, and a wavefront issues one
+//    instruction at a time (k_march_mixed 55.5 -> 50 us at 1024 x 1500, together
+//    with the tables in FP32; k_tile 27.9 -> 27.4 at 512 x 512).  Lanes whose
+//    column lies before the array wrap the 32-bit offset; they are the masked
+//    halo lanes and access nothing.
+//  * the row's 64-bit address, pinned to SGPRs (readfirstlane of a uniform
+//    value), plus the lane offset: the mixed marching body's for fields of
+//    4 GiB or more.
+// Both go through a global-address-space pointer, so the accesses stay
 // global_load / global_store (a generic pointer made from an integer would
 // compile to flat accesses, which also count against the LDS wait counter).
 template <typename T>
 using GlobalBytes =
     __attribute__((address_space(1))) typename std::conditional<std::is_const<T>::value, const char, char>::type;
+
+template <typename T>
+__device__ __forceinline__ T& lane_at(T* row, unsigned loff) {
+  const unsigned long long u = (unsigned long long)row;
+  const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)u);
+  const unsigned hi = __builtin_amdgcn_readfirstlane((unsigned)(u >> 32));
+  GlobalBytes<T>* base = (GlobalBytes<T>*)(((unsigned long long)hi << 32) | lo);
+  return *(T*)(base + loff);
+}
 
 template <typename T>
 struct RowRef {

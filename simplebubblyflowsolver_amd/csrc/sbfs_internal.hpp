@@ -177,10 +177,16 @@ int npy_write(const char* dir, const char* name, const char* descr,
               const std::vector<size_t>& shape, size_t elem, const void* data);
 int load_dt_coefs();
 
-// The FP64 stage kernels address a field by its base and a 32-bit byte
+// The stage kernels address a field by its base and a 32-bit byte
 // offset (march.hip): every field of the grid, the vof with its two halo
-// rows on each side the largest, must stay below 4 GiB.
+// rows on each side the largest, must stay below 4 GiB.  Larger FP64 grids take the
+// staged path, larger mixed ones the mixed kernels with 64-bit row addresses
+// (SBFS_MARCH_WIDE=1 forces those; the results are bitwise the same).
 inline bool fp64_march_addressable(size_t nx, size_t ny) { return (ny + 4) * (nx + 2) * 8 < (1ull << 32); }
+inline bool mixed_march_wide(size_t nx, size_t ny) {
+  const char* e = getenv("SBFS_MARCH_WIDE");
+  return (e && e[0] == '1') || !fp64_march_addressable(nx, ny);
+}
 // Whether the single-case kernels stream the rows they touch once
 // (non-temporal loads and stores): only when an FP64 field outgrows what the
 // 256 MB Infinity Cache keeps between one kernel and the next; below that,
