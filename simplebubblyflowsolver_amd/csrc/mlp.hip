@@ -387,6 +387,17 @@ constexpr int kGradST = 2;               // subtiles per tile
 constexpr int kGradS = 16 * kGradST;     // samples per tile
 constexpr int kGradWaves = 4 * kGradST;  // wavefronts per tile
 
+// x % n for x >= 0, n > 0.  Below 2^52 by an FP64 quotient, which is off by one at
+// most: the 64-bit remainder's 150 instructions stand before the tile's first load
+// (k_mlp_grad 9.3 -> 9.1 us between events).
+__device__ __forceinline__ long sample_index(long x, long n) {
+  if (x >= (1l << 52)) return x % n;
+  long r = x - (long)((double)x / (double)n) * n;
+  if (r < 0) r += n;
+  if (r >= n) r -= n;
+  return r;
+}
+
 template <int ST>
 __global__ __launch_bounds__(256 * ST) void k_mlp_grad(Weights w, const unsigned short* __restrict__ X,
                                                        const float* __restrict__ T, const float* __restrict__ Wt,
@@ -412,7 +423,7 @@ __global__ __launch_bounds__(256 * ST) void k_mlp_grad(Weights w, const unsigned
   // per sample, 2 features each
   {
     const int sm = t >> 4, fp = t & 15;
-    const long idx = (first + (tile * S + sm) * stride) % n;
+    const long idx = sample_index(first + (tile * S + sm) * stride, n);
     const unsigned v = *(const unsigned*)(X + (size_t)idx * NIP + 2 * fp);
     *(unsigned*)(sx + sm * XP + 2 * fp) = v;
     sxt[(2 * fp) * SP + sm] = (unsigned short)(v & 0xFFFFu);
@@ -567,16 +578,20 @@ struct AdamState {
   unsigned short* w2tb;
 };
 
-// A workgroup of 256 threads takes 32 parameters, 8 threads each: thread
-// `sl` sums the tiles [sl tiles / 8, (sl + 1) tiles / 8) in order, 16 loads
-// in flight at a time, and the first thread adds the 8 slice sums in order.
-constexpr int kAdamSlices = 8;
-__global__ __launch_bounds__(256) void k_mlp_adam(AdamState s, const float* __restrict__ part, int tiles, int adam,
+// A workgroup takes 64 parameters, a wavefront each of their 8 slices: thread
+// (sl, pk) sums the tiles [sl tiles / 8, (sl + 1) tiles / 8) of parameter pk in
+// order, 16 loads in flight at a time and 256 bytes of a tile per wavefront, and
+// the first wavefront adds the 8 slice sums in order.  A step at batch 4096 is
+// bound by the latency of its two launches; 100 workgroups instead of 198 with 8
+// slices per wavefront (32 bytes of a tile each) took it from 13.0 to 11.7 us,
+// 32 or 128 parameters to 12.1 and 11.6.
+constexpr int kAdamSlices = 8, kAdamParams = 64;
+__global__ __launch_bounds__(kAdamParams * kAdamSlices) void k_mlp_adam(AdamState s, const float* __restrict__ part, int tiles, int adam,
                                                   float lr, float b1t, float b2t, float* __restrict__ grad,
                                                   float* __restrict__ loss) {
-  __shared__ float slice[256];
-  const int sl = (int)threadIdx.x % kAdamSlices;
-  const int k = (int)blockIdx.x * (256 / kAdamSlices) + (int)threadIdx.x / kAdamSlices;
+  __shared__ float slice[kAdamSlices][kAdamParams];
+  const int sl = (int)threadIdx.x / kAdamParams, pk = (int)threadIdx.x % kAdamParams;
+  const int k = (int)blockIdx.x * kAdamParams + pk;
   const int t1 = (int)(((long)tiles * (sl + 1)) / kAdamSlices);
   int t = (int)(((long)tiles * sl) / kAdamSlices);
   float gs = 0.f;
@@ -590,12 +605,12 @@ __global__ __launch_bounds__(256) void k_mlp_adam(AdamState s, const float* __re
     }
     for (; t < t1; t++) gs += part[(size_t)t * NPART + k];
   }
-  slice[threadIdx.x] = gs;
+  slice[sl][pk] = gs;
   __syncthreads();
   if (sl != 0 || k > NP) return;
   float g = 0.f;
 #pragma unroll
-  for (int u = 0; u < kAdamSlices; u++) g += slice[threadIdx.x + u];
+  for (int u = 0; u < kAdamSlices; u++) g += slice[u][pk];
   if (grad) grad[k] = g;
   if (k == NP) {
     if (loss) *loss = g;
@@ -1105,7 +1120,7 @@ extern "C" int sbfs_mlp_gradient(const float* features, const float* targets, co
   SBFS_HIP(hipMemcpyAsync(s.w, hw.data(), sizeof(float) * n, hipMemcpyHostToDevice, stream()));
   int rc = grad_pass(s, 0, 1, tiles, 2.f / (float)n, part);
   if (!rc) {
-    hipLaunchKernelGGL(k_mlp_adam, dim3(cdiv(NPART * kAdamSlices, 256)), dim3(256), 0, stream(), adam_state(), (const float*)part,
+    hipLaunchKernelGGL(k_mlp_adam, dim3(cdiv(NPART, kAdamParams)), dim3(kAdamParams * kAdamSlices), 0, stream(), adam_state(), (const float*)part,
                        tiles, 0, 0.f, 1.f, 1.f, g, (float*)nullptr);
     rc = check_launch("sbfs_mlp_gradient");
   }
@@ -1195,7 +1210,7 @@ extern "C" int sbfs_mlp_train(uint64_t seed, size_t nsamples, int epochs, int ba
       const float b1t = 1.f - powf(0.9f, (float)g_net.step), b2t = 1.f - powf(0.999f, (float)g_net.step);
       rc = grad_pass(s, offset + k * batch * stride, stride, tiles, 2.f / (float)batch, part);
       if (!rc) {
-        SBFS_TIMED("k_mlp_adam", hipLaunchKernelGGL(k_mlp_adam, dim3(cdiv(NPART * kAdamSlices, 256)), dim3(256), 0, stream(),
+        SBFS_TIMED("k_mlp_adam", hipLaunchKernelGGL(k_mlp_adam, dim3(cdiv(NPART, kAdamParams)), dim3(kAdamParams * kAdamSlices), 0, stream(),
                                                     adam_state(), (const float*)part, tiles, 1, lrk, b1t, b2t,
                                                     (float*)nullptr, loss + e * steps + k));
         rc = check_launch("sbfs_mlp_train");
