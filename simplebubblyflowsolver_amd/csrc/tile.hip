@@ -17,9 +17,11 @@
 //   5  predicted velocity, the rows' outputs             density, curvature, tyy s-1
 //   6  Poisson right-hand side                           face terms s+1
 //
-// Rows jb-2 .. je+3 are needed for output rows jb .. je.  Columns, lanes, masks
+// Rows jb-2 .. je+3 are needed for output rows jb .. je; a wavefront ends before
+// the first phase that needs nothing of its row (a barrier waits for the ones
+// that remain: k_tile at 512 x 512 28.5 -> 27.6 us).  Columns, lanes, masks
 // and every expression are the marching kernel's, so the fields are the same bit
-// for bit.  The latency of the seven phases bounds it (119 VGPRs in FP64, 93 in
+// for bit.  The latency of the seven phases bounds it (121 VGPRs in FP64, 98 in
 // FP32: 4 and 5 wavefronts per SIMD, but one workgroup of H = 11 fills a CU's LDS
 // by half), so the marching kernel keeps the grids where the device is full.
 // The three stages together, us with about 15 of the timing events:
