@@ -764,7 +764,7 @@ static int fused_body(const domain_t* domain, DomainCtx* c, fluid_t* fluid, inte
         m.order = scr.order;
         m.weight = scr.weight;
       }
-      const dim3 grid = ordered ? dim3(units) : dim3(cdiv(nx, kStrip), cdiv(ny, band)), block(64);
+      const dim3 grid = ordered ? dim3(cdiv(units, 8 * kOrderChunk) * 8 * kOrderChunk) : dim3(cdiv(nx, kStrip), cdiv(ny, band)), block(64);
       const MarchArgs* ma = nullptr;
       if (device_args(c, m, &ma)) return 1;
       if (tile) {

@@ -772,13 +772,24 @@ __global__ __launch_bounds__(1024) void k_march_order(const unsigned* __restrict
 // overlap by 6 columns and share their end lines, run on one XCD and read them from
 // its L2.  Dealt out in turn, each XCD fetched them again: k_march_mixed 930 -> 763
 // us and folded 1180 -> 948 at 4096 x 8192, 213 -> 186 and 285 -> 249 at 2048 x 4096,
-// 49 -> 47 and 63 -> 60 at 1024 x 1500.
+// 49 -> 47 and 63 -> 60 at 1024 x 1500.  In the dispatch order, whose units of equal
+// weight are mostly neighbours too, an XCD takes runs of kOrderChunk entries of each
+// 8 kOrderChunk: k_march 1076 -> 1048 us and folded 1424 -> 1394 at 4096 x 8192,
+// 286 -> 285 and 362 -> 356 at 2048 x 4096, 99.5 -> 98 and 120.5 -> 119.4 at
+// 1024 x 2048.  (Runs of 64 gave 350 at 2048 x 4096 but 122 at 1024 x 2048; of 128,
+// where the heaviest no longer start first, 418 and 149.  Without the order, eighths
+// as above and three rounds took 4000 us instead of 3880 for a step's three at
+// 4096 x 8192.)
 __device__ __forceinline__ bool march_unit(const MarchArgs& a, int& bx, int& by) {
   bx = blockIdx.x;
   by = blockIdx.y;
   if (a.order) {
-    const unsigned u = (unsigned)__builtin_amdgcn_readfirstlane((int)a.order[blockIdx.x]);
-    if (u >= (unsigned)march_units(a.nx, a.ny, a.band)) return false;
+    const unsigned b = blockIdx.x, n = (unsigned)march_units(a.nx, a.ny, a.band);
+    constexpr unsigned C = kOrderChunk;
+    const unsigned at = b / (8 * C) * (8 * C) + b % 8 * C + b / 8 % C;
+    if (at >= n) return false;
+    const unsigned u = (unsigned)__builtin_amdgcn_readfirstlane((int)a.order[at]);
+    if (u >= n) return false;
     const int strips = march_strips(a.nx);
     bx = (int)u % strips;
     by = (int)u / strips;

@@ -22,6 +22,9 @@ constexpr int kStrip = 58;
 // match with the staged one.)
 constexpr int kWarm = 4;
 constexpr int kWarmCorr = 4;
+// consecutive entries of the dispatch order on one XCD (march_unit); the grid is
+// rounded up to whole rounds of 8 XCDs
+constexpr int kOrderChunk = 16;
 // Output rows of a workgroup of the small grids' stage kernel (tile.hip): the
 // short tile has the shorter latency, the tall one less redundant work.
 constexpr int kTileShort = 3, kTileTall = 11;
