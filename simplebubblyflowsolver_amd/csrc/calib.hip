@@ -32,8 +32,8 @@ extern "C" int sbfs_copy_bandwidth(size_t bytes, int reps, double* gbs) {
   SBFS_REQUIRE(bytes >= 16 && bytes % 16 == 0, "bytes must be a positive multiple of 16");
   const size_t n = bytes / 16;
   double2 *src = nullptr, *dst = nullptr;
-  SBFS_HIP(hipMalloc(&src, bytes));
-  SBFS_HIP(hipMalloc(&dst, bytes));
+  SBFS_HIP(device_malloc(&src, bytes));
+  SBFS_HIP(device_malloc(&dst, bytes));
   int rc = 0;
   hipEvent_t e0 = nullptr, e1 = nullptr;
   do {

@@ -217,7 +217,7 @@ static int plan(sbfs_ensemble* e) {
   }
   e->nb_post = (unsigned)map.size() - e->off_post;
   e->lds = lds_rows;
-  SBFS_HIP(hipMalloc(&e->maps, sizeof(uint2) * map.size()));
+  SBFS_HIP(device_malloc(&e->maps, sizeof(uint2) * map.size()));
   SBFS_HIP(hipMemcpy(e->maps, map.data(), sizeof(uint2) * map.size(), hipMemcpyHostToDevice));
   for (int p = 0; p < 2; p++) {
     std::vector<DtArgs> dt(n);
@@ -232,10 +232,10 @@ static int plan(sbfs_ensemble* e) {
         ro[(size_t)k * n + c] = steps[p][c].rows[k];
       }
     }
-    SBFS_HIP(hipMalloc(&e->dt[p], sizeof(DtArgs) * n));
-    SBFS_HIP(hipMalloc(&e->march[p], sizeof(MarchArgs) * ma.size()));
-    SBFS_HIP(hipMalloc(&e->rows[p], sizeof(RowArgs) * ro.size()));
-    SBFS_HIP(hipMalloc(&e->post[p], sizeof(PostArgs) * n));
+    SBFS_HIP(device_malloc(&e->dt[p], sizeof(DtArgs) * n));
+    SBFS_HIP(device_malloc(&e->march[p], sizeof(MarchArgs) * ma.size()));
+    SBFS_HIP(device_malloc(&e->rows[p], sizeof(RowArgs) * ro.size()));
+    SBFS_HIP(device_malloc(&e->post[p], sizeof(PostArgs) * n));
     SBFS_HIP(hipMemcpy(e->dt[p], dt.data(), sizeof(DtArgs) * n, hipMemcpyHostToDevice));
     SBFS_HIP(hipMemcpy(e->march[p], ma.data(), sizeof(MarchArgs) * ma.size(), hipMemcpyHostToDevice));
     SBFS_HIP(hipMemcpy(e->rows[p], ro.data(), sizeof(RowArgs) * ro.size(), hipMemcpyHostToDevice));
@@ -341,7 +341,7 @@ static int snapshot(sbfs_ensemble* e, std::vector<void*>& save, bool restore) {
     for (array_t* a : arrs) {
       if (!restore) {
         void* b = nullptr;
-        SBFS_HIP(hipMalloc(&b, a->datasize));
+        SBFS_HIP(device_malloc(&b, a->datasize));
         SBFS_HIP(hipMemcpyAsync(b, a->data, a->datasize, hipMemcpyDeviceToDevice, stream()));
         save.push_back(b);
       } else {
@@ -382,7 +382,7 @@ extern "C" int sbfs_ensemble_create(const sbfs_case_t* cases, int n, sbfs_ensemb
       const size_t sizes[] = {k.s.vof.datasize, k.f.ux.datasize, k.f.ux.datasize,
                               k.f.uy.datasize,  k.f.uy.datasize, k.f.p.datasize};
       for (int b = 0; b < 6 && !rc; b++) {
-        if (hipMalloc(bufs[b], sizes[b]) != hipSuccess ||
+        if (device_malloc(bufs[b], sizes[b]) != hipSuccess ||
             hipMemsetAsync(*bufs[b], 0, sizes[b], stream()) != hipSuccess) {
           set_error("sbfs_ensemble_create: out of device memory");
           rc = 1;

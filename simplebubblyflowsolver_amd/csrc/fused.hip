@@ -19,8 +19,6 @@
 #include <cstdint>
 #include <cstdlib>
 #include <cstring>
-#include <mutex>
-#include <utility>
 #include <vector>
 
 #include "decide_dt.h"
@@ -31,6 +29,7 @@
 #include "poisson.hpp"
 #include "sbfs.h"
 #include "sbfs_internal.hpp"
+#include "scratch_pool.hpp"
 #include "stencils.hpp"
 
 namespace sbfs {
@@ -201,25 +200,6 @@ __global__ __launch_bounds__(256) void k_post_batch(const PostArgs* __restrict__
 // ---------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------
-struct FusedScratch {
-  size_t nx = 0, ny = 0;
-  double* vof = nullptr;
-  double* ux = nullptr;   // predicted velocity of stages 0 and 2
-  double* uy = nullptr;
-  double* ux2 = nullptr;  // predicted velocity of stage 1 (folded projection)
-  double* uy2 = nullptr;
-  double* p = nullptr;    // pressure written by a stage kernel with the folded projection
-  // learned curvature only (allocated when it is first used):
-  float* kappa = nullptr;  // learned curvature of a stage's input vof (interior cells)
-  unsigned* klist[3] = {};  // its listed cells (count first), one list per stage
-  int klast = -1;            // the list of the last launch (-1: none since the fill)
-  unsigned long long* cut = nullptr;  // cut-cell bitmask of a stage kernel's new vof
-  // the stage kernels' dispatch order and unit weights (march.hpp)
-  unsigned* weight = nullptr;
-  unsigned* order = nullptr;
-  int units = 0;
-};
-
 struct CoefTables {
   double re = 0.;
   double* buf = nullptr;
@@ -267,21 +247,21 @@ struct FusedState {
   uint64_t clock = 0;
 };
 
-static void scratch_free(FusedScratch& s) {
-  for (double* q : {s.vof, s.ux, s.uy, s.ux2, s.uy2, s.p}) (void)hipFree(q);
-  (void)hipFree(s.kappa);
-  for (unsigned* l : s.klist) (void)hipFree(l);
-  (void)hipFree(s.cut);
-  (void)hipFree(s.weight);
-  (void)hipFree(s.order);
-  s = FusedScratch();
-}
+struct DeviceMemory {
+  static int alloc(void** p, size_t bytes) {
+    const hipError_t e = hipMalloc(p, bytes);
+    if (e != hipSuccess) {
+      *p = nullptr;
+      (void)hipGetLastError();  // (a later launch check would report it)
+    }
+    return e;
+  }
+  static void free(void* p) { (void)hipFree(p); }
+  static int zero(void* p, size_t bytes) { return hipMemsetAsync(p, 0, bytes, stream()); }
+};
+static ScratchPool<DeviceMemory> g_pool;
 
-// The scratch of the last domain given back, for the next one of its size: a
-// program that closes a case and opens another allocates no scratch.  One set
-// at most.
-static std::mutex g_spare_mutex;
-static FusedScratch g_spare;
+hipError_t device_malloc_bytes(void** p, size_t bytes) { return (hipError_t)g_pool.alloc(p, bytes); }
 
 // (the caller has synchronised the stream)
 void fused_destroy(FusedState* s) {
@@ -290,51 +270,30 @@ void fused_destroy(FusedState* s) {
     if (g.exec) (void)hipGraphExecDestroy(g.exec);
   (void)hipFree(s->coef.buf);
   (void)hipFree(s->args_dev);
-  if (s->scr.vof) {
-    std::lock_guard<std::mutex> lock(g_spare_mutex);
-    scratch_free(g_spare);
-    g_spare = s->scr;
-  }
+  g_pool.put(s->scr);
   delete s;
 }
 
 static int scratch(DomainCtx* c, const interface_t* s, const fluid_t* f, bool learned) {
   FusedScratch& scr = c->fused->scr;
   const size_t cells = c->nx * c->ny;
-  if (!scr.vof) {
-    {
-      std::lock_guard<std::mutex> lock(g_spare_mutex);
-      if (g_spare.vof && g_spare.nx == c->nx && g_spare.ny == c->ny) {
-        scr = g_spare;
-        g_spare = FusedScratch();
-      }
-    }
-    if (!scr.vof) {
-      const std::pair<double**, size_t> bufs[] = {{&scr.ux, f->ux.datasize},   {&scr.uy, f->uy.datasize},
-                                                  {&scr.ux2, f->ux.datasize},  {&scr.uy2, f->uy.datasize},
-                                                  {&scr.p, f->p.datasize},     {&scr.vof, s->vof.datasize}};
-      // (the vof last: it marks the set as whole)
-      for (const auto& b : bufs) {
-        (void)hipFree(*b.first);
-        *b.first = nullptr;
-        double* q = nullptr;
-        SBFS_HIP(hipMalloc(&q, b.second));
-        const hipError_t e = hipMemsetAsync(q, 0, b.second, stream());
-        if (e != hipSuccess) (void)hipFree(q);
-        SBFS_HIP(e);
-        *b.first = q;
-      }
-      scr.nx = c->nx;
-      scr.ny = c->ny;
-    }
-  }
+  if (!scr.vof)
+    SBFS_HIP((hipError_t)g_pool.get(
+        {c->nx, c->ny, f->ux.datasize, f->uy.datasize, f->p.datasize, s->vof.datasize}, learned, &scr));
   if (learned && !scr.cut) {
-    if (!scr.kappa) SBFS_HIP(hipMalloc(&scr.kappa, sizeof(float) * cells));
+    // (what a failed call here allocated stays in the set)
+    auto part = [&scr](auto** p, size_t bytes) -> int {
+      if (*p) return 0;
+      SBFS_HIP(device_malloc(p, bytes));
+      scr.bytes += bytes;
+      return 0;
+    };
+    if (part(&scr.kappa, sizeof(float) * cells)) return 1;
     for (unsigned*& l : scr.klist)
-      if (!l) SBFS_HIP(hipMalloc(&l, sizeof(unsigned) * (cells + 1)));
+      if (part(&l, sizeof(unsigned) * (cells + 1))) return 1;
     if (curv_field_init(scr.kappa, scr.klist, 3, (long)cells, stream())) return 1;
     scr.klast = -1;
-    SBFS_HIP(hipMalloc(&scr.cut, sizeof(unsigned long long) * c->ny * march_strips((int)c->nx)));
+    if (part(&scr.cut, sizeof(unsigned long long) * c->ny * march_strips((int)c->nx))) return 1;
   }
   return 0;
 }
@@ -349,8 +308,8 @@ static int order_buffers(DomainCtx* c, int n) {
   (void)hipFree(scr.order);
   scr.weight = scr.order = nullptr;
   scr.units = 0;
-  SBFS_HIP(hipMalloc(&scr.weight, sizeof(unsigned) * (size_t)n));
-  SBFS_HIP(hipMalloc(&scr.order, sizeof(unsigned) * (size_t)n));
+  SBFS_HIP(device_malloc(&scr.weight, sizeof(unsigned) * (size_t)n));
+  SBFS_HIP(device_malloc(&scr.order, sizeof(unsigned) * (size_t)n));
   SBFS_HIP(hipMemsetAsync(scr.weight, 0, sizeof(unsigned) * (size_t)n, stream()));
   scr.units = n;
   return 0;
@@ -385,7 +344,7 @@ int coef_build(const domain_t* d, double Re, double** buf, Coef* out) {
     t[11][i] = diffusivity / jc;
     t[13][i] = hc;
   }
-  SBFS_HIP(hipMalloc(buf, sizeof(double) * h.size()));
+  SBFS_HIP(device_malloc(buf, sizeof(double) * h.size()));
   SBFS_HIP(hipMemcpy(*buf, h.data(), sizeof(double) * h.size(), hipMemcpyHostToDevice));
   const double* b = *buf;
   Coef cf;
@@ -659,7 +618,7 @@ static int device_args(DomainCtx* c, const MarchArgs& m, const MarchArgs** out) 
   SBFS_HIP(hipStreamIsCapturing(stream(), &cs));
   SBFS_REQUIRE(cs == hipStreamCaptureStatusNone,
                "integrate: stage arguments of a captured step were not prepared by its eager pass");
-  if (!s.args_dev) SBFS_HIP(hipMalloc(&s.args_dev, sizeof(MarchArgs) * kMaxArgSlots));
+  if (!s.args_dev) SBFS_HIP(device_malloc(&s.args_dev, sizeof(MarchArgs) * kMaxArgSlots));
   if (s.args.size() >= kMaxArgSlots) {
     // captured graphs hold pointers to these slots: move the epoch so that
     // none of them replays (queued steps read them before the stores below)

@@ -132,7 +132,7 @@ extern "C" int sbfs_logging_values(const domain_t* domain, const fluid_t* fluid,
   const int nx = (int)c->nx, ny = (int)c->ny;
   static double* buf = nullptr;  // partials + result, grown once
   constexpr int kBlocks = 1024;
-  if (!buf) SBFS_HIP(hipMalloc(&buf, sizeof(double) * (size_t)Q_N * (kBlocks + 1)));
+  if (!buf) SBFS_HIP(device_malloc(&buf, sizeof(double) * (size_t)Q_N * (kBlocks + 1)));
   LogArgs a;
   a.vof = (const double*)interface->vof.data;
   a.ux = (const double*)fluid->ux.data;

@@ -921,10 +921,10 @@ static Net g_net;
 
 static int net_alloc() {
   if (g_net.p) return 0;
-  SBFS_HIP(hipMalloc(&g_net.p, sizeof(float) * NP * 3));
+  SBFS_HIP(device_malloc(&g_net.p, sizeof(float) * NP * 3));
   g_net.m = g_net.p + NP;
   g_net.v = g_net.p + 2 * NP;
-  SBFS_HIP(hipMalloc(&g_net.w1b, sizeof(unsigned short) * (NH * NIP + 2 * NH * NH)));
+  SBFS_HIP(device_malloc(&g_net.w1b, sizeof(unsigned short) * (NH * NIP + 2 * NH * NH)));
   g_net.w2b = g_net.w1b + NH * NIP;
   g_net.w2tb = g_net.w2b + NH * NH;
   // on the library stream (non-blocking): a null-stream memset is not
@@ -984,8 +984,8 @@ struct Samples {
 
 static int make_samples(uint64_t seed, long n, Samples& s) {
   SBFS_REQUIRE(n > 0, "mlp: no samples");
-  SBFS_HIP(hipMalloc(&s.x, sizeof(unsigned short) * NIP * (size_t)n));
-  SBFS_HIP(hipMalloc(&s.t, sizeof(float) * 2 * (size_t)n));
+  SBFS_HIP(device_malloc(&s.x, sizeof(unsigned short) * NIP * (size_t)n));
+  SBFS_HIP(device_malloc(&s.t, sizeof(float) * 2 * (size_t)n));
   s.w = s.t + n;
   s.n = n;
   s.seed = seed;
@@ -1053,9 +1053,9 @@ extern "C" int sbfs_mlp_samples(uint64_t seed, size_t first, size_t n, float* fe
   SBFS_REQUIRE(n > 0 && features && labels, "sbfs_mlp_samples: bad arguments");
   unsigned short* x = nullptr;
   float *t = nullptr, *f = nullptr;
-  SBFS_HIP(hipMalloc(&x, sizeof(unsigned short) * NIP * n));
-  SBFS_HIP(hipMalloc(&t, sizeof(float) * 3 * n));
-  if (stencils) SBFS_HIP(hipMalloc(&f, sizeof(float) * NI * n));
+  SBFS_HIP(device_malloc(&x, sizeof(unsigned short) * NIP * n));
+  SBFS_HIP(device_malloc(&t, sizeof(float) * 3 * n));
+  if (stencils) SBFS_HIP(device_malloc(&f, sizeof(float) * NI * n));
   hipLaunchKernelGGL(k_mlp_samples, dim3(cdiv((long)n, 128)), dim3(128), 0, stream(), seed, (long)first, (long)n,
                      x, t + n, t + 2 * n, t, f);
   int rc = check_launch("sbfs_mlp_samples");
@@ -1107,14 +1107,14 @@ extern "C" int sbfs_mlp_gradient(const float* features, const float* targets, co
   std::vector<float> hw(n, 1.f);
   if (weights) memcpy(hw.data(), weights, sizeof(float) * n);
   Samples s;
-  SBFS_HIP(hipMalloc(&s.x, sizeof(unsigned short) * NIP * n));
-  SBFS_HIP(hipMalloc(&s.t, sizeof(float) * 2 * n));
+  SBFS_HIP(device_malloc(&s.x, sizeof(unsigned short) * NIP * n));
+  SBFS_HIP(device_malloc(&s.t, sizeof(float) * 2 * n));
   s.w = s.t + n;
   s.n = (long)n;
   const int tiles = (int)(n / kGradS);
   float *part = nullptr, *g = nullptr;
-  SBFS_HIP(hipMalloc(&part, sizeof(float) * NPART * tiles));
-  SBFS_HIP(hipMalloc(&g, sizeof(float) * NPART));
+  SBFS_HIP(device_malloc(&part, sizeof(float) * NPART * tiles));
+  SBFS_HIP(device_malloc(&g, sizeof(float) * NPART));
   SBFS_HIP(hipMemcpyAsync(s.x, hx.data(), sizeof(unsigned short) * NIP * n, hipMemcpyHostToDevice, stream()));
   SBFS_HIP(hipMemcpyAsync(s.t, targets, sizeof(float) * n, hipMemcpyHostToDevice, stream()));
   SBFS_HIP(hipMemcpyAsync(s.w, hw.data(), sizeof(float) * n, hipMemcpyHostToDevice, stream()));
@@ -1154,8 +1154,8 @@ extern "C" int sbfs_mlp_predict(const double* stencils, size_t n, double* out) {
   }
   unsigned short* x = nullptr;
   float* y = nullptr;
-  SBFS_HIP(hipMalloc(&x, sizeof(unsigned short) * NIP * n));
-  SBFS_HIP(hipMalloc(&y, sizeof(float) * n));
+  SBFS_HIP(device_malloc(&x, sizeof(unsigned short) * NIP * n));
+  SBFS_HIP(device_malloc(&y, sizeof(float) * n));
   SBFS_HIP(hipMemcpyAsync(x, hx.data(), sizeof(unsigned short) * NIP * n, hipMemcpyHostToDevice, stream()));
   hipLaunchKernelGGL(k_mlp_predict, dim3(cdiv((long)n, 64)), dim3(64), 0, stream(), weights(), x, (long)n, y);
   int rc = check_launch("sbfs_mlp_predict");
@@ -1186,8 +1186,8 @@ extern "C" int sbfs_mlp_train(uint64_t seed, size_t nsamples, int epochs, int ba
   const int tiles = batch / kGradS;
   const long steps = (long)(nsamples / (size_t)batch);
   float *part = nullptr, *loss = nullptr;
-  SBFS_HIP(hipMalloc(&part, sizeof(float) * NPART * tiles));
-  SBFS_HIP(hipMalloc(&loss, sizeof(float) * steps * epochs));
+  SBFS_HIP(device_malloc(&part, sizeof(float) * NPART * tiles));
+  SBFS_HIP(device_malloc(&loss, sizeof(float) * steps * epochs));
   int rc = 0;
   const long n = (long)nsamples;
   for (int e = 0; e < epochs && !rc; e++) {
@@ -1257,9 +1257,9 @@ extern "C" int sbfs_mlp_coverage(const domain_t* domain, const interface_t* inte
   float* k = nullptr;
   unsigned* list = nullptr;
   unsigned long long* cnt = nullptr;
-  SBFS_HIP(hipMalloc(&k, sizeof(float) * n));
-  SBFS_HIP(hipMalloc(&list, sizeof(unsigned) * (n + 1)));
-  SBFS_HIP(hipMalloc(&cnt, sizeof(unsigned long long)));
+  SBFS_HIP(device_malloc(&k, sizeof(float) * n));
+  SBFS_HIP(device_malloc(&list, sizeof(unsigned) * (n + 1)));
+  SBFS_HIP(device_malloc(&cnt, sizeof(unsigned long long)));
   SBFS_HIP(hipMemsetAsync(cnt, 0, sizeof(unsigned long long), stream()));
   int rc = curv_field_init(k, &list, 1, n, stream());
   if (!rc)

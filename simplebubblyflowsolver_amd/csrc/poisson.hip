@@ -822,10 +822,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
 static int sequential_setup(PoissonPlan* p, double l) {
   if (p->cl) return 0;
   const size_t cells = (size_t)p->nx * p->ny;
-  if (!p->v) SBFS_HIP(hipMalloc(&p->v, sizeof(double) * cells));
-  if (!p->q1) SBFS_HIP(hipMalloc(&p->q1, sizeof(double) * cells));
+  if (!p->v) SBFS_HIP(device_malloc(&p->v, sizeof(double) * cells));
+  if (!p->q1) SBFS_HIP(device_malloc(&p->q1, sizeof(double) * cells));
   double* cl = nullptr;
-  SBFS_HIP(hipMalloc(&cl, sizeof(double) * p->nx));
+  SBFS_HIP(device_malloc(&cl, sizeof(double) * p->nx));
   if (tdm_columns(p->ny)) {
     hipLaunchKernelGGL(k_tdm_factors, dim3(cdiv(p->nx, 64)), dim3(64), 0, stream(), p->v, p->q1, cl, p->nx, p->ny,
                        p->evals, l, l);
@@ -925,11 +925,11 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2))) void k
 // ---------------------------------------------------------------------------
 static int plan_build(PoissonPlan* p, const domain_t* d) {
   const int nx = p->nx, ny = p->ny, m = p->m;
-  SBFS_HIP(hipMalloc(&p->buf, sizeof(double) * (size_t)nx * ny));
-  SBFS_HIP(hipMalloc(&p->evals, sizeof(double) * nx));
-  SBFS_HIP(hipMalloc(&p->tw, sizeof(double2) * (m > 0 ? m : 1)));
-  SBFS_HIP(hipMalloc(&p->t1, sizeof(double2) * (m + 1)));
-  SBFS_HIP(hipMalloc(&p->t2, sizeof(double2) * nx));
+  SBFS_HIP(device_malloc(&p->buf, sizeof(double) * (size_t)nx * ny));
+  SBFS_HIP(device_malloc(&p->evals, sizeof(double) * nx));
+  SBFS_HIP(device_malloc(&p->tw, sizeof(double2) * (m > 0 ? m : 1)));
+  SBFS_HIP(device_malloc(&p->t1, sizeof(double2) * (m + 1)));
+  SBFS_HIP(device_malloc(&p->t2, sizeof(double2) * nx));
   // eigenvalues of the x operator, compute_potential.c:233-261
   std::vector<double> ev(nx);
   const double sl = 2. * (double)d->glsizes[0];
@@ -1045,7 +1045,7 @@ static int poisson_tail(const domain_t* d, PoissonPlan* p, fluid_t* f) {
 int poisson_transform_fused(const domain_t* d, DomainCtx* c, fluid_t* f, double** rhs_out) {
   PoissonPlan* p = plan_get(d, c);
   if (!p) return 1;
-  if (!p->rhs) SBFS_HIP(hipMalloc(&p->rhs, sizeof(double) * (size_t)p->nx * p->ny));
+  if (!p->rhs) SBFS_HIP(device_malloc(&p->rhs, sizeof(double) * (size_t)p->nx * p->ny));
   if (rhs_out) {
     *rhs_out = p->rhs;
     return 0;
@@ -1071,7 +1071,7 @@ int poisson_transform_fused(const domain_t* d, DomainCtx* c, fluid_t* f, double*
 int poisson_row_args(const domain_t* d, DomainCtx* c, double* psi, RowArgs* a) {
   PoissonPlan* p = plan_get(d, c);
   if (!p) return 1;
-  if (!p->rhs) SBFS_HIP(hipMalloc(&p->rhs, sizeof(double) * (size_t)p->nx * p->ny));
+  if (!p->rhs) SBFS_HIP(device_malloc(&p->rhs, sizeof(double) * (size_t)p->nx * p->ny));
   a->rhs = p->rhs;
   a->buf = p->buf;
   SBFS_REQUIRE(((uintptr_t)psi & 15) == 0, "poisson: psi[1] must be 16-byte aligned (hipMalloc'ed)");
@@ -1129,11 +1129,11 @@ extern "C" int sbfs_dct_rows(int inverse, size_t n, size_t howmany, const double
   double *din = nullptr, *dout = nullptr;
   double2 *dtw = nullptr, *dt1 = nullptr, *dt2 = nullptr;
   const size_t bytes = sizeof(double) * n * howmany;
-  SBFS_HIP(hipMalloc(&din, bytes));
-  SBFS_HIP(hipMalloc(&dout, bytes));
-  SBFS_HIP(hipMalloc(&dtw, sizeof(double) * tw.size()));
-  SBFS_HIP(hipMalloc(&dt1, sizeof(double) * t1.size()));
-  SBFS_HIP(hipMalloc(&dt2, sizeof(double) * t2.size()));
+  SBFS_HIP(device_malloc(&din, bytes));
+  SBFS_HIP(device_malloc(&dout, bytes));
+  SBFS_HIP(device_malloc(&dtw, sizeof(double) * tw.size()));
+  SBFS_HIP(device_malloc(&dt1, sizeof(double) * t1.size()));
+  SBFS_HIP(device_malloc(&dt2, sizeof(double) * t2.size()));
   SBFS_HIP(hipMemcpy(din, in_host, bytes, hipMemcpyHostToDevice));
   SBFS_HIP(hipMemcpy(dtw, tw.data(), sizeof(double) * tw.size(), hipMemcpyHostToDevice));
   SBFS_HIP(hipMemcpy(dt1, t1.data(), sizeof(double) * t1.size(), hipMemcpyHostToDevice));

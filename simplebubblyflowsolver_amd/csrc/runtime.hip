@@ -228,13 +228,13 @@ DomainCtx* domain_ctx(const domain_t* d) {
   c->ly = d->lengths[1];
   c->hy = d->hy;
   c->hash = h;
-  bool ok = hipMalloc(&c->hxxf, sizeof(double) * (nx + 1)) == hipSuccess &&
-            hipMalloc(&c->hxxc, sizeof(double) * nx) == hipSuccess &&
-            hipMalloc(&c->jdxf, sizeof(double) * (nx + 1)) == hipSuccess &&
-            hipMalloc(&c->jdxc, sizeof(double) * nx) == hipSuccess &&
-            hipMalloc(&c->xc, sizeof(double) * (nx + 2)) == hipSuccess &&
-            hipMalloc(&c->red, sizeof(double) * kRedSlots) == hipSuccess &&
-            hipMalloc(&c->dt, sizeof(DtSlot)) == hipSuccess &&
+  bool ok = device_malloc(&c->hxxf, sizeof(double) * (nx + 1)) == hipSuccess &&
+            device_malloc(&c->hxxc, sizeof(double) * nx) == hipSuccess &&
+            device_malloc(&c->jdxf, sizeof(double) * (nx + 1)) == hipSuccess &&
+            device_malloc(&c->jdxc, sizeof(double) * nx) == hipSuccess &&
+            device_malloc(&c->xc, sizeof(double) * (nx + 2)) == hipSuccess &&
+            device_malloc(&c->red, sizeof(double) * kRedSlots) == hipSuccess &&
+            device_malloc(&c->dt, sizeof(DtSlot)) == hipSuccess &&
             hipMemset(c->dt, 0, sizeof(DtSlot)) == hipSuccess &&
             hipHostMalloc(&c->host_pin, sizeof(double) * 16, 0) == hipSuccess;
   if (!ok || upload_metrics(d, c)) {
@@ -307,7 +307,7 @@ static int prepare(const domain_t* d, const Nadds& na, size_t elem, array_t* a) 
   }
   a->datasize = nxt * nyt * elem;
   a->data = nullptr;
-  SBFS_HIP(hipMalloc(&a->data, a->datasize));
+  SBFS_HIP(device_malloc(&a->data, a->datasize));
   SBFS_HIP(hipMemsetAsync(a->data, 0, a->datasize, g_stream));
   return 0;
 }

@@ -168,6 +168,13 @@ hipStream_t side_stream();
 hipEvent_t fork_event(int k);
 hipEvent_t join_event(int k);
 int init_runtime();
+// hipMalloc for all of the library: where it fails, the scratch kept for the
+// next domains (fused.hip) is freed and it is tried again
+hipError_t device_malloc_bytes(void** p, size_t bytes);
+template <typename T>
+inline hipError_t device_malloc(T** p, size_t bytes) {
+  return device_malloc_bytes((void**)p, bytes);
+}
 // device context of a host domain (created / refreshed on demand)
 DomainCtx* domain_ctx(const domain_t* d);
 

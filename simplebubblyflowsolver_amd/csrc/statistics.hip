@@ -36,9 +36,9 @@ static int stats_prepare(const domain_t* d) {
   (void)hipFree(g_stats.uy1);
   (void)hipFree(g_stats.vof1);
   g_stats = Stats();
-  SBFS_HIP(hipMalloc(&g_stats.ux1, sizeof(double) * (nx + 1) * ny));
-  SBFS_HIP(hipMalloc(&g_stats.uy1, sizeof(double) * (nx + 2) * ny));
-  SBFS_HIP(hipMalloc(&g_stats.vof1, sizeof(double) * (nx + 2) * ny));
+  SBFS_HIP(device_malloc(&g_stats.ux1, sizeof(double) * (nx + 1) * ny));
+  SBFS_HIP(device_malloc(&g_stats.uy1, sizeof(double) * (nx + 2) * ny));
+  SBFS_HIP(device_malloc(&g_stats.vof1, sizeof(double) * (nx + 2) * ny));
   SBFS_HIP(hipMemsetAsync(g_stats.ux1, 0, sizeof(double) * (nx + 1) * ny, stream()));
   SBFS_HIP(hipMemsetAsync(g_stats.uy1, 0, sizeof(double) * (nx + 2) * ny, stream()));
   SBFS_HIP(hipMemsetAsync(g_stats.vof1, 0, sizeof(double) * (nx + 2) * ny, stream()));

@@ -359,10 +359,10 @@ int partition_setup(PoissonPlan* p, const domain_t* d, int L) {
     host_periodic_tdm(P, lo, di, up, pin, hcol.data(), hv.data(), hq1.data());
     for (int c = 0; c < P; c++) htab[(size_t)c * nx + mo] = hcol[c];
   }
-  SBFS_HIP(hipMalloc(&p->ptab, sizeof(double) * tab.size()));
-  SBFS_HIP(hipMalloc(&p->gfl, sizeof(double) * 2 * (size_t)P * nx));
-  SBFS_HIP(hipMalloc(&p->X, sizeof(double) * (size_t)P * nx));
-  SBFS_HIP(hipMalloc(&p->htab, sizeof(double) * htab.size()));
+  SBFS_HIP(device_malloc(&p->ptab, sizeof(double) * tab.size()));
+  SBFS_HIP(device_malloc(&p->gfl, sizeof(double) * 2 * (size_t)P * nx));
+  SBFS_HIP(device_malloc(&p->X, sizeof(double) * (size_t)P * nx));
+  SBFS_HIP(device_malloc(&p->htab, sizeof(double) * htab.size()));
   SBFS_HIP(hipMemcpy(p->htab, htab.data(), sizeof(double) * htab.size(), hipMemcpyHostToDevice));
   SBFS_HIP(hipMemcpy(p->ptab, tab.data(), sizeof(double) * tab.size(), hipMemcpyHostToDevice));
   p->L = L;
