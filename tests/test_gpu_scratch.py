@@ -34,16 +34,3 @@ def test_a_large_case_gives_its_scratch_back(product):
         assert held < 0.3e9
     finally:
         c.close()
-
-
-def test_sets_of_several_sizes_come_back(product):
-    """Cases of three sizes opened and closed in turn, twice over: the second
-    time no device memory is taken that the first did not leave."""
-    def round_():
-        cs = [step_once(product, nx, ny) for nx, ny in ((64, 128), (256, 256), (512, 100), (256, 256))]
-        for c in cs:
-            c.close()
-        return free_bytes(product)
-
-    first = round_()
-    assert all(round_() >= first - (1 << 21) for _ in range(3))
