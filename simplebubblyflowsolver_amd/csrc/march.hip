@@ -36,7 +36,9 @@ namespace sbfs {
 // LDS of one wavefront: the column tables, and the older rows that the folded
 // FP32 body keeps there (it has no VGPRs left for them; each lane reads back
 // only what it wrote, so no barrier is needed).  The FP64 body has: with them
-// in LDS its folded kernel took 355 us instead of 352 at 2048 x 4096.
+// in LDS a step takes 1485 us instead of 1479 at 2048 x 4096 and 570 instead of
+// 567 at 1024 x 2048 with diagnostics; at 4096 x 8192 the two are level (5918 to
+// 5937 and 5921 to 5950).
 enum { RG_QUXS, RG_CYCUYS, RG_D1X, RG_CGY, RG_PSM1, RG_PM1, RG_DNM1, RG_N };
 // The FP32 body's FP64 tables are the four that its FP64 parts read (fp64_slot).
 template <typename R>
@@ -765,6 +767,7 @@ __global__ __launch_bounds__(1024) void k_march_order(const unsigned* __restrict
 // MarchArgs outgrow the scalar registers, and the compiler spills them into
 // vector lanes (v_writelane / v_readlane in the row loop, up to 185 of them
 // in the FP64 folded body); from memory it reloads them with scalar loads.
+
 // the (strip, band) of this workgroup: from the grid, or from the dispatch
 // order (false: a slot past the last unit)
 // In the grid's order, XCD x (the hardware deals workgroups to the 8 XCDs in turn)
@@ -774,12 +777,13 @@ __global__ __launch_bounds__(1024) void k_march_order(const unsigned* __restrict
 // us and folded 1180 -> 948 at 4096 x 8192, 213 -> 186 and 285 -> 249 at 2048 x 4096,
 // 49 -> 47 and 63 -> 60 at 1024 x 1500.  In the dispatch order, whose units of equal
 // weight are mostly neighbours too, an XCD takes runs of kOrderChunk entries of each
-// 8 kOrderChunk: k_march 1076 -> 1048 us and folded 1424 -> 1394 at 4096 x 8192,
-// 286 -> 285 and 362 -> 356 at 2048 x 4096, 99.5 -> 98 and 120.5 -> 119.4 at
-// 1024 x 2048.  (Runs of 64 gave 350 at 2048 x 4096 but 122 at 1024 x 2048; of 128,
-// where the heaviest no longer start first, 418 and 149.  Without the order, eighths
-// as above and three rounds took 4000 us instead of 3880 for a step's three at
-// 4096 x 8192.)
+// 8 kOrderChunk: an FP64 step 1524 -> 1488 us at 2048 x 4096 (k_march 261 -> 260 and
+// folded 346 -> 333), 6007 -> 5962 at 4096 x 8192 with the bubbles on a regular
+// pattern and level with them at random (5947 and 5948); k_march 99.5 -> 98 and folded
+// 120.5 -> 119.4 at 1024 x 2048.  (Runs of 64 took the folded kernel from 356 to 350
+// at 2048 x 4096 but from 119 to 122 at 1024 x 2048; of 128, where the heaviest no
+// longer start first, to 418 and 149.  Without the order, eighths as above and three
+// rounds took 4000 us instead of 3880 for a step's three at 4096 x 8192.)
 __device__ __forceinline__ bool march_unit(const MarchArgs& a, int& bx, int& by) {
   bx = blockIdx.x;
   by = blockIdx.y;
@@ -807,9 +811,10 @@ __device__ __forceinline__ bool march_unit(const MarchArgs& a, int& bx, int& by)
 // without the walls' lane masks.  In the masked body about 170 exec-mask blocks
 // with their branches interrupt a row step, which every strip paid for the few
 // at the walls; without them k_march takes 264 us instead of 283 at 2048 x 4096
-// and 1102 instead of 1175 at 4096 x 8192, with the fold 338 instead of 347 and
-// 1414 instead of 1450.  The FP32 bodies, which wait for memory more than they
-// compute, got slower (2048 x 4096: 206 us against 198, with the fold 273 against 261)
+// and the folded kernel 333 instead of 352.  At 4096 x 8192, where the card's power
+// bounds the FP64 step, the folded kernel's inner body takes the step from 6004 to
+// 5950 us with the bubbles on a regular pattern and is level with them at random (5913
+// and 5925).  The FP32 bodies, which wait for memory more than they compute, got slower (2048 x 4096: 206 us against 198, with the fold 273 against 261)
 // and keep the one masked body.
 __device__ __forceinline__ bool march_inner(int nx, int bx) { return bx >= 1 && 1 + bx * kStrip + 60 <= nx; }
 template <typename R, bool CORR, bool ALT>
