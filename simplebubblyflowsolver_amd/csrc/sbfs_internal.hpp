@@ -109,6 +109,7 @@ struct FusedState;   // fused.hip
 // decide_dt's result on the device and the words its workgroups combine their
 // minima in (step.hip), which are 0 between launches
 constexpr unsigned kDtWords = 32, kDtFlat = 128;
+constexpr int kDtMaxGx = 8192;  // groups of kRedThreads columns that decide_dt takes
 struct alignas(128) DtWord {
   unsigned long long key;
   unsigned count;

@@ -156,8 +156,7 @@ int dt_args(const domain_t* d, const DomainCtx* c, const fluid_t* f, const inter
   a->nx = (int)c->nx;
   a->ny = (int)c->ny;
   a->gx = (int)cdiv(a->nx, kRedThreads);
-  SBFS_REQUIRE(a->gx <= kRedBlocks * 8, "decide_dt: %d columns need %d partial minima, more than the %d slots", a->nx,
-               a->gx, kRedBlocks * 8);
+  SBFS_REQUIRE(a->gx <= kDtMaxGx, "decide_dt: %d columns, more than %d", a->nx, kDtMaxGx * kRedThreads);
   a->rows = 4;
   while (a->gx * cdiv(a->ny, a->rows) > 2048 && a->rows < 64) a->rows *= 2;
   a->nblk = a->gx * (int)cdiv(a->ny, a->rows);
