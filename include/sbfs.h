@@ -225,9 +225,11 @@ extern int sbfs_ensemble_case(sbfs_ensemble_t * ensemble, int k,
                               interface_t ** interface);
 /* one step of every case; dts[k] (may be null) receives case k's dt */
 extern int sbfs_ensemble_step(sbfs_ensemble_t * ensemble, double * dts);
-/* band height of the stage kernel (rows per wavefront; default 32):
+/* band height of the marching stage kernel (rows per wavefront; default 32):
  * autotune times every candidate on the ensemble's current state, restores
- * it and keeps the fastest; both need an even number of steps taken */
+ * it and keeps the fastest; both need an even number of steps taken.  Small
+ * ensembles take a stage kernel without bands: autotune then runs no trial and
+ * returns the band as it is. */
 extern int sbfs_ensemble_autotune(sbfs_ensemble_t * ensemble, int * band);
 extern int sbfs_ensemble_set_band(sbfs_ensemble_t * ensemble, int band);
 extern int sbfs_ensemble_destroy(sbfs_ensemble_t * ensemble);

@@ -10,9 +10,10 @@
 // second time it runs.  Per case the step is the single-case fused step with
 // the projection folded and the tridiagonal algorithm the options select
 // for that case (partitioned or sequential), so a case run in an ensemble
-// gives the same bits as the case run alone.  The band height of the stage kernel
-// is the only tile shape the ensemble chooses; sbfs_ensemble_autotune times
-// the candidates on the ensemble itself.
+// gives the same bits as the case run alone.  Small ensembles take the stage
+// kernel of small grids, by the rule of a single case (tile_rows); for the others
+// the marching kernel's band height is the only tile shape that is open, and
+// sbfs_ensemble_autotune times the candidates on the ensemble itself.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -428,6 +429,12 @@ extern "C" int sbfs_ensemble_autotune(sbfs_ensemble_t* e, int* band) {
   // the one restored
   if (e->planned && e->parity != 0) {
     SBFS_REQUIRE(false, "sbfs_ensemble_autotune: call it after an even number of steps");
+  }
+  // a small ensemble's stage kernel has no bands
+  if (plan(e)) return 1;
+  if (e->tile) {
+    if (band) *band = e->band;
+    return 0;
   }
   std::vector<void*> save;
   if (snapshot(e, save, false)) return 1;
