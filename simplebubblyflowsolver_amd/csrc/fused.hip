@@ -865,9 +865,11 @@ static int step_graph(const domain_t* domain, DomainCtx* c, fluid_t* fluid, inte
   bool seen = false;
   for (const StepKey& k : fs.seen) seen = seen || k == key;
   if (!seen) {
-    // first sight of this configuration: run eagerly (builds plans / tables)
-    fs.seen[fs.clock % kStepGraphs] = key;
-    return fused_body(domain, c, fluid, interface, cf, rhs, band, learned_h);
+    // first sight of this configuration: run eagerly (builds plans / tables);
+    // one that failed has not built them all, and the next one runs eagerly too
+    const int rc = fused_body(domain, c, fluid, interface, cf, rhs, band, learned_h);
+    if (!rc) fs.seen[fs.clock % kStepGraphs] = key;
+    return rc;
   }
   StepGraph* slot = &fs.graph[0];
   for (StepGraph& g : fs.graph)
