@@ -723,17 +723,22 @@ static int fused_body(const domain_t* domain, DomainCtx* c, fluid_t* fluid, inte
         m.order = scr.order;
         m.weight = scr.weight;
       }
-      const dim3 grid = ordered ? dim3(cdiv(units, 8 * kOrderChunk) * 8 * kOrderChunk) : dim3(cdiv(nx, kStrip), cdiv(ny, band)), block(64);
+      const dim3 block(64), grid = ordered ? dim3(cdiv(units, 8 * kOrderChunk) * 8 * kOrderChunk)
+                                           : dim3(cdiv(nx, kStrip), cdiv(ny, band));
       const MarchArgs* ma = nullptr;
       if (device_args(c, m, &ma)) return 1;
       if (tile) {
         tile_launch(ma, nx, ny, tile, mixed, corr);
       } else if (mixed && corr)
-        SBFS_TIMED("k_march_mixed_corr", hipLaunchKernelGGL((wide ? k_march_mixed_corr_wide : k_march_mixed_corr), grid, block, 0, stream(), ma));
+        SBFS_TIMED("k_march_mixed_corr",
+                   hipLaunchKernelGGL((wide ? k_march_mixed_corr_wide : k_march_mixed_corr), grid, block, 0, stream(),
+                                      ma));
       else if (mixed)
-        SBFS_TIMED("k_march_mixed", hipLaunchKernelGGL((wide ? k_march_mixed_wide : k_march_mixed), grid, block, 0, stream(), ma));
+        SBFS_TIMED("k_march_mixed",
+                   hipLaunchKernelGGL((wide ? k_march_mixed_wide : k_march_mixed), grid, block, 0, stream(), ma));
       else if (corr)
-        SBFS_TIMED("k_march_corr", hipLaunchKernelGGL((nt ? k_march_corr_nt : k_march_corr), grid, block, 0, stream(), ma));
+        SBFS_TIMED("k_march_corr",
+                   hipLaunchKernelGGL((nt ? k_march_corr_nt : k_march_corr), grid, block, 0, stream(), ma));
       else
         SBFS_TIMED("k_march", hipLaunchKernelGGL((nt ? k_march_nt : k_march), grid, block, 0, stream(), ma));
       if (check_launch("integrate: k_march")) return 1;
@@ -779,7 +784,7 @@ static int fused_body(const domain_t* domain, DomainCtx* c, fluid_t* fluid, inte
 // Graph replay of the fused step.  The step's launches depend only on the
 // array pointers, the case parameters and the options, and the pointers
 // return to one of two states (psi and vof swap an odd number of times per
-// step), so up to two captured graphs serve a run.  A configuration is
+// step), so two captured graphs serve a run and a domain keeps four.  A configuration is
 // captured the second time it is seen: the first, eager, pass builds every
 // plan and table the step needs, so the captured sequence allocates and
 // synchronises nothing.  Profiling (per-launch events) and SBFS_GRAPH=0

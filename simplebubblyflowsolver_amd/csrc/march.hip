@@ -19,9 +19,10 @@
 //
 // Older rows stay in register rings, x-neighbours come from DPP wavefront
 // shifts, so nothing is recomputed across rows and no LDS tile or barrier is
-// needed; a term shared by two neighbouring faces or rows is formed once.  Every value is formed with the reference's operation order (the
-// per-column quotients come from the coefficient tables), which keeps the
-// result bitwise equal to the staged kernels.
+// needed; a term shared by two neighbouring faces or rows is formed once.  Every
+// value is formed with the reference's operation order (the per-column quotients
+// come from the coefficient tables), which keeps the result bitwise equal to the
+// staged kernels.
 #include "march_dev.hpp"
 
 #ifndef SBFS_FP64_WAVES
@@ -814,8 +815,9 @@ __device__ __forceinline__ bool march_unit(const MarchArgs& a, int& bx, int& by)
 // and the folded kernel 333 instead of 352.  At 4096 x 8192, where the card's power
 // bounds the FP64 step, the folded kernel's inner body takes the step from 6004 to
 // 5950 us with the bubbles on a regular pattern and is level with them at random (5913
-// and 5925).  The FP32 bodies, which wait for memory more than they compute, got slower (2048 x 4096: 206 us against 198, with the fold 273 against 261)
-// and keep the one masked body.
+// and 5925).  The FP32 bodies, which wait for memory more than they compute, got
+// slower (2048 x 4096: 206 us against 198, with the fold 273 against 261) and keep the
+// one masked body.
 __device__ __forceinline__ bool march_inner(int nx, int bx) { return bx >= 1 && 1 + bx * kStrip + 60 <= nx; }
 template <typename R, bool CORR, bool ALT>
 __device__ __forceinline__ void march_strip(const MarchArgs& a, int bx, int by) {

@@ -842,7 +842,11 @@ static int sequential_solve(PoissonPlan* p, double l, int pin) {
   if (sequential_setup(p, l)) return 1;
   const int nx = p->nx, ny = p->ny, mw = tdm_columns(ny);
   const size_t lds = tdm_column_lds(ny, mw);
-#define SBFS_COLUMNS(MW)                                                                                            SBFS_TIMED("k_tdm_columns", hipLaunchKernelGGL(k_tdm_columns<MW>, dim3(cdiv(nx, MW)), dim3(256), lds, stream(),                                                  p->buf, (const double*)p->v, (const double*)p->q1,                                                                (const double*)p->cl, nx, ny, (const double*)p->evals, l, l, pin))
+#define SBFS_COLUMNS(MW)                                                                                       \
+  SBFS_TIMED("k_tdm_columns",                                                                                  \
+             hipLaunchKernelGGL(k_tdm_columns<MW>, dim3(cdiv(nx, MW)), dim3(256), lds, stream(), p->buf,       \
+                                (const double*)p->v, (const double*)p->q1, (const double*)p->cl, nx, ny,       \
+                                (const double*)p->evals, l, l, pin))
   if (mw == 4) SBFS_COLUMNS(4);
   else if (mw == 2) SBFS_COLUMNS(2);
   else if (mw == 1) SBFS_COLUMNS(1);
@@ -890,7 +894,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
   const uint2 mp = map[blockIdx.x];
   const RowArgs& a = tab[mp.x];
   switch (tdm_columns(a.ny)) {
-#define SBFS_COLUMN_CASE(MW)   case MW: tdm_column_body<MW>(a.buf, a.v, a.q1, a.cl, a.nx, a.ny, a.evals, a.l, a.l, a.pin, (int)mp.y * MW, col); break
+#define SBFS_COLUMN_CASE(MW)                                                                                   \
+  case MW:                                                                                                     \
+    tdm_column_body<MW>(a.buf, a.v, a.q1, a.cl, a.nx, a.ny, a.evals, a.l, a.l, a.pin, (int)mp.y * MW, col);    \
+    break
     SBFS_COLUMN_CASE(4);
     SBFS_COLUMN_CASE(2);
     SBFS_COLUMN_CASE(1);
