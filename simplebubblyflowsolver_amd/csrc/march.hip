@@ -37,9 +37,11 @@ namespace sbfs {
 // LDS of one wavefront: the column tables, and the older rows that the folded
 // FP32 body keeps there (it has no VGPRs left for them; each lane reads back
 // only what it wrote, so no barrier is needed).  The FP64 body has: with them
-// in LDS a step takes 1485 us instead of 1479 at 2048 x 4096 and 570 instead of
-// 567 at 1024 x 2048 with diagnostics; at 4096 x 8192 the two are level (5918 to
-// 5937 and 5921 to 5950).
+// in LDS a step takes 1484 us instead of 1480 at 2048 x 4096 and 569 instead of
+// 566 at 1024 x 2048 with diagnostics.  The streaming one, of larger grids, keeps
+// them in LDS all the same: at 4096 x 8192 a step takes 5931 us (5916 to 5949)
+// instead of 5957 (5923 to 5986) with the bubbles at random, 5947 instead of 5974
+// on a regular pattern (eight runs each, after 60 steps).
 enum { RG_QUXS, RG_CYCUYS, RG_D1X, RG_CGY, RG_PSM1, RG_PM1, RG_DNM1, RG_N };
 // The FP32 body's FP64 tables are the four that its FP64 parts read (fp64_slot).
 template <typename R>
@@ -53,8 +55,8 @@ struct MarchLds {
   float sf[kSingle ? T_N : 1][64];
   double rings[LR ? RG_N : 1][64];
 };
-template <typename R, bool CORR>
-constexpr bool kLdsRings = CORR && std::is_same<R, float>::value;
+template <typename R, bool CORR, bool ALT>
+constexpr bool kLdsRings = CORR && (std::is_same<R, float>::value || ALT);
 
 // R = double: the plain FP64 step.  R = float: the stencils of the
 // interface (gradients, normals, curvature, THINC and mass fluxes) and of the
@@ -68,7 +70,7 @@ constexpr bool kLdsRings = CORR && std::is_same<R, float>::value;
 // FP32 ones address rows by 64 bits (see row below)
 template <typename R, bool CORR, bool ALT, bool IN>
 __device__ __forceinline__ void march_body(const MarchArgs& a, int bx, int by,
-                                           MarchLds<R, kLdsRings<R, CORR>>& lds) {
+                                           MarchLds<R, kLdsRings<R, CORR, ALT>>& lds) {
   using A = Arith<R>;
   using V3 = V3R<R>;
   constexpr bool NT = ALT && std::is_same<R, double>::value, WIDE = ALT && std::is_same<R, float>::value;
@@ -105,7 +107,7 @@ __device__ __forceinline__ void march_body(const MarchArgs& a, int bx, int by,
     for (int t = 0; t < T_N; t++) tab[t] = tabs[t][cc];
   }
   const double dt_in = *a.dt;
-  constexpr bool LR = kLdsRings<R, CORR>;
+  constexpr bool LR = kLdsRings<R, CORR, ALT>;
   const int ll = lane > 0 ? lane - 1 : 0, lr = lane < 63 ? lane + 1 : 63;
   // tables in FP64 (the FP64 parts) and in the stencil type
   // (those in FP32 are rounded once here: converted at each use they cost 20
@@ -779,8 +781,8 @@ __global__ __launch_bounds__(1024) void k_march_order(const unsigned* __restrict
 // 49 -> 47 and 63 -> 60 at 1024 x 1500.  In the dispatch order, whose units of equal
 // weight are mostly neighbours too, an XCD takes runs of kOrderChunk entries of each
 // 8 kOrderChunk: an FP64 step 1524 -> 1488 us at 2048 x 4096 (k_march 261 -> 260 and
-// folded 346 -> 333), 6007 -> 5962 at 4096 x 8192 with the bubbles on a regular
-// pattern and level with them at random (5947 and 5948); k_march 99.5 -> 98 and folded
+// folded 346 -> 333), 6006 -> 5950 at 4096 x 8192 with the bubbles on a regular
+// pattern and level with them at random (5934 and 5925); k_march 99.5 -> 98 and folded
 // 120.5 -> 119.4 at 1024 x 2048.  (Runs of 64 took the folded kernel from 356 to 350
 // at 2048 x 4096 but from 119 to 122 at 1024 x 2048; of 128, where the heaviest no
 // longer start first, to 418 and 149.  Without the order, eighths as above and three
@@ -821,7 +823,7 @@ __device__ __forceinline__ bool march_unit(const MarchArgs& a, int& bx, int& by)
 __device__ __forceinline__ bool march_inner(int nx, int bx) { return bx >= 1 && 1 + bx * kStrip + 60 <= nx; }
 template <typename R, bool CORR, bool ALT>
 __device__ __forceinline__ void march_strip(const MarchArgs& a, int bx, int by) {
-  __shared__ MarchLds<R, kLdsRings<R, CORR>> lds;
+  __shared__ MarchLds<R, kLdsRings<R, CORR, ALT>> lds;
   if (std::is_same<R, double>::value && march_inner(a.nx, bx)) march_body<R, CORR, ALT, true>(a, bx, by, lds);
   else march_body<R, CORR, ALT, false>(a, bx, by, lds);
 }
